@@ -46,6 +46,10 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // estimate of the launch (band_shrinks).
 constexpr int64_t kMinShrunkBandRows = 8;
 constexpr int kMaxShrink = 6;
+// No matrix is shrunk past this many bands: few workgroups add its partials per column (eight for 2048 columns), and
+// at 2000 bands of 32000x2048 that took 72 us twice a step.
+constexpr int64_t kMaxShrunkBands = 512;
+constexpr int64_t kFactorFewBlocks = 512;  // a factor launch of at most this many blocks takes eight wavefronts a block
 constexpr int64_t kMinLaunchBands = 2048;  // without a device to ask: the least work items per launch
 // Fixed time of a band (its start, its row sums, its partial stores), about 5 us, in elements the
 // whole GPU streams meanwhile: a workgroup among `slots` spends it as kBandFixedElems / slots.
@@ -59,6 +63,7 @@ int64_t band_rows(int64_t R, int64_t C, int shrink = 0) {
   int64_t rb = std::max<int64_t>(1, (int64_t(1) << 20) / std::max<int64_t>(C, 1));
   rb = std::min<int64_t>(rb, kMaxBandRows);
   rb = std::max<int64_t>(std::min<int64_t>(rb, kMinShrunkBandRows), rb >> shrink);
+  rb = std::max<int64_t>(rb, std::min<int64_t>(kMaxBandRows, ceil_div(R, kMaxShrunkBands)));
   return std::min<int64_t>(rb, R);
 }
 
@@ -103,8 +108,9 @@ struct Plan {
   std::map<BandKey, WorkList> bandN;     // P1 of the default clip mode, the same tensors (k_fact_pass1n; st = 1)
   std::map<BandKey, WorkList> band2dw;   // P1 of the 8bit2d tensors (both modes: their clip takes W)
   std::map<BandKey, WorkList> band2;     // P2 (factored tensors of the full8bit / fp32 layouts)
-  std::map<int, WorkList> tiny1;         // P1 of tensors of tiny matrices (per 256 matrices), by grad type
+  std::map<int, WorkList> tiny1;         // P1 of tensors of tiny matrices (per ngrp matrices), by grad type
   std::map<int, WorkList> tiny2;         // P2 of tensors of tiny matrices, by grad type
+  WorkList tinyq;                        // their states' codes (per four state blocks)
   std::map<TypeKey, WorkList> upd;       // P3, tile form (fast block sizes)
   std::map<TypeKey, WorkList> updb;      // P3, band form
   std::map<TypeKey, WorkList> vecB;      // 1-D pass B (fast block sizes)
@@ -228,6 +234,9 @@ void magic_div(int64_t d, uint64_t& m, uint32_t& s) {
 bool tiny_matrix(const came8_tensor& t, bool s2d) {
   return t.factored && !s2d && t.rows >= 1 && t.cols >= 1 && t.rows * t.cols <= kTinyElems;
 }
+
+// Matrices per work item of those passes, and per unit of the clip-norm estimates (at most kNormMaxUnits of them)
+int64_t tiny_group(int64_t P) { return kThreads * ceil_div(P, int64_t(kThreads) * kNormMaxUnits); }
 
 // The clip-norm estimate of a tensor takes a workgroup per row band (matrices at least a workgroup
 // wide) rather than a thread per unit.
@@ -487,9 +496,12 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
       d.nbands = ceil_div(d.R, d.rb);
       d.nbr = d.pm ? d.P * d.pmb_r : std::max<int64_t>(1, ceil_div(d.P * d.R, B));
       d.nbc = d.pm ? d.P * d.pmb_c : std::max<int64_t>(1, ceil_div(d.P * d.C, B));
-      d.nclip = d.nbc;
+      const bool tiny = tiny_matrix(t, s2d);
+      // the thread-per-matrix passes write a clip partial (and norm estimate) per work item
+      const int64_t tiny_items = ceil_div(d.P, tiny_group(d.P));
+      d.nclip = tiny ? tiny_items : d.nbc;
       const size_t pr = size_t(d.P * d.R) * 4, pc = size_t(d.P * d.C) * 4;
-      const size_t part = size_t(d.P * d.nbands * d.C) * 4;
+      const size_t part = tiny ? 0 : size_t(d.P * d.nbands * d.C) * 4;  // (they keep no column partials)
       o.Rn = take(pr); o.rfac = take(pr); o.RRn = take(pr); o.rrfac = take(pr);
       o.Cn = take(pc); o.cfac = take(pc); o.CRn = take(pc); o.crfac = take(pc);
       o.pU = take(part); o.pW = take(part);
@@ -531,8 +543,9 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
       // 256 such runs takes shorter ones, down to 16, so that it still spreads over the CUs
       d.nrun = d.nseg0 >= 256 * int64_t(kNormRunSegs) ? kNormRunSegs : (d.nseg0 >= 128 * int64_t(kNormRunSegs) ? 32 : 16);
       const int64_t nbase = t.factored ? d.P * d.nbands : d.nclip;
+      if (tiny_matrix(t, false)) d.ngrp = tiny_group(d.P);
       // the thread-per-unit estimate groups single-band matrices and tiles into at most kNormMaxUnits units
-      if (!norm_est_wide(t, d) && (!t.factored || d.nbands == 1)) d.ngrp = ceil_div(nbase, kNormMaxUnits);
+      else if (!norm_est_wide(t, d) && (!t.factored || d.nbands == 1)) d.ngrp = ceil_div(nbase, kNormMaxUnits);
       d.nunit = ceil_div(nbase, d.ngrp);
       o.nest = take(size_t(d.nunit + 1) * 4);
       o.nrec = take(size_t(d.nseg) * 3 * 8 * 4);
@@ -630,8 +643,9 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     }
     if (t.factored) {
       if (tiny_matrix(t, false)) {
-        add_item(plan.tiny1[t.grad_dtype], i, ceil_div(d.P, int64_t(kThreads)));
-        add_item((longc[i] ? plan.tiny2L : plan.tiny2)[t.grad_dtype], i, ceil_div(d.P, int64_t(kThreads)));
+        add_item(plan.tiny1[t.grad_dtype], i, d.nclip);
+        add_item((longc[i] ? plan.tiny2L : plan.tiny2)[t.grad_dtype], i, d.nclip);
+        if (!d.fp32st) add_item(plan.tinyq, i, ceil_div(d.nbr + d.nbc, int64_t(4)));
       } else {
         const bool pm_m = d.pm && (d.R * d.C) % B != 0;
         const BandShapeSel sel1 = band_variant(t, d.C, B, 1), sel2 = band_variant(t, d.C, B, 2, pm_m);
@@ -643,7 +657,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
         add_item((longc[i] ? plan.band2L : plan.band2)[BandKey{t.grad_dtype, sel2.V, sel2.K, sel2.TPB, d.fp32st, sel2.ua,
                                                               sel2.multiseg}], i, d.P * d.nbands);
       }
-      add_item(plan.factor, i, d.nbr + d.nbc);
+      if (!tiny_matrix(t, false)) add_item(plan.factor, i, d.nbr + d.nbc);
       // per-matrix momentum blocks that end inside a matrix (B does not divide R*C) are not the flat
       // passes' blocks: such tensors take the per-block kernel
       const bool pm_odd = d.pm && (d.R * d.C) % B != 0;
@@ -664,7 +678,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     // one segment needs no estimates, records or rebuild.
     if (d.nseg > 1) {
       if (norm_est_wide(t, d)) add_item(plan.nest_w, i, d.nunit);
-      else add_item(plan.nest_n, i, ceil_div(d.nunit, int64_t(kThreads)));
+      else if (!tiny_matrix(t, false)) add_item(plan.nest_n, i, ceil_div(d.nunit, int64_t(kThreads)));
       // the vector forms need rows of whole aligned 8-element chunks and 32-bit flat indices; matrices
       // (prefix 1) up to kNormLdsCols wide take runs of segments with their column factors in LDS
       const bool vec = t.factored && d.idx32 && reinterpret_cast<uintptr_t>(t.grad) % 16 == 0;
@@ -699,6 +713,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
   for (auto& kv : plan.param2d_b) place(kv.second);
   for (auto& kv : plan.param2d) place(kv.second);
   place(plan.res2d);
+  place(plan.tinyq);
   for (auto& kv : plan.upd) place(kv.second);
   for (auto& kv : plan.updb) place(kv.second);
   for (auto& kv : plan.vecB) place(kv.second);
@@ -773,6 +788,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     for (auto& kv : plan.param2d_b) put(kv.second);
     for (auto& kv : plan.param2d) put(kv.second);
     put(plan.res2d);
+    put(plan.tinyq);
     for (auto& kv : plan.upd) put(kv.second);
     for (auto& kv : plan.updb) put(kv.second);
     for (auto& kv : plan.vecB) put(kv.second);
@@ -1434,6 +1450,18 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     }
     return CAME8_OK;
   };
+  // LDS of a thread-per-matrix pass: its largest matrices
+  auto tiny_bytes = [&](const WorkList& wl, bool codes) {
+    size_t bytes = 0;
+    for (int32_t ti : wl.tids) bytes = std::max(bytes, tiny_lds(plan.dev[ti].R * plan.dev[ti].C, codes));
+    return bytes;
+  };
+  auto launch_state_quant = [&](auto kernel, const char* what) -> int {
+    if (plan.tinyq.tids.empty()) return CAME8_OK;
+    const WorkList& wl = plan.tinyq;
+    hipLaunchKernelGGL(kernel, dim3(grid_for(wl.total())), blk, 0, stream, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
+    return check_launch(what);
+  };
   // P2 of one group of factored tensors: through the pass's queues, or all on queue q
   auto launch_pass2 = [&](const std::map<BandKey, WorkList>& bands, const std::map<int, WorkList>& tinies,
                           bool via_pq, hipStream_t q) -> int {
@@ -1459,10 +1487,18 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
       if (!via_pq) ls = q;
       else if ((r = pq.pick(ab, &ls)) != CAME8_OK) return r;
       PhaseTimer pt(PH_PASS2, ab, ls);
-      hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), blk, 0, ls, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
+      hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), blk, tiny_bytes(wl, true), ls, dT, tids(wl), wst(wl),
+                         int(wl.tids.size()), hp);
       if ((r = check_launch("tiny_pass2")) != CAME8_OK) return r;
     }
     return CAME8_OK;
+  };
+  // Factor kernels: eight wavefronts share a block's band sums while the launch has few blocks, else four (a lone
+  // 2048x2048 in 256 bands: 14.5 + 12.9 -> 10.9 + 10.8 us; 1745 blocks of 292 tensors: four 22.6, eight 36.7 us)
+  auto launch_factor = [&](auto kernel4, auto kernel8, const WorkList& wl, size_t lds4, size_t lds8) {
+    const bool few = wl.total() <= kFactorFewBlocks;
+    hipLaunchKernelGGL(few ? kernel8 : kernel4, dim3(grid_for(wl.total())), dim3((few ? 8 : 4) * kWave),
+                       few ? lds8 : lds4, stream, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
   };
   bool split = false;  // the long-chain group runs on the side stream (set by the clip-norm section)
 
@@ -1493,7 +1529,8 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     const double ab = alg_bytes(plan, wl, tensors, PH_PASS1);
     if ((rc = pq.pick(ab, &ls)) != CAME8_OK) return rc;
     { PhaseTimer pt(PH_PASS1, ab, ls);
-    hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), blk, 0, ls, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
+    hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), blk, tiny_bytes(wl, false), ls, dT, tids(wl), wst(wl),
+                       int(wl.tids.size()), hp);
     if ((rc = check_launch("tiny_pass1")) != CAME8_OK) return rc; }
   }
   for (auto& kv : vecA) {
@@ -1507,14 +1544,17 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     if ((rc = check_launch("vec_passA")) != CAME8_OK) return rc; }
   }
   if ((rc = pq.finish()) != CAME8_OK) return rc;
-  const bool any_fact = !plan.factor.tids.empty();
-  if (any_fact) {
+  const bool any_factor = !plan.factor.tids.empty();
+  const bool any_fact = any_factor || !plan.tiny1.empty();
+  const bool any2d = !plan.tiles2d.empty() || !plan.tiles2d_v.empty();
+  if (any_factor) {
     const WorkList& fb = plan.factor;
     { PhaseTimer pt(PH_FACTOR, alg_bytes(plan, fb, tensors, PH_FACTOR), stream);
-    hipLaunchKernelGGL(k_factor_blocks<false>, dim3(grid_for(fb.total())), blk, 0, stream, dT, tids(fb), wst(fb),
-                       int(fb.tids.size()), hp);
+    launch_factor(k_factor_blocks<false, 4>, k_factor_blocks<false, 8>, fb, factor_lds(4, exact_norm || any2d),
+                  factor_lds(8, exact_norm || any2d));
     if ((rc = check_launch("factor_blocks")) != CAME8_OK) return rc; }
   }
+  if ((rc = launch_state_quant(k_state_quant<false>, "state_quant")) != CAME8_OK) return rc;
   // ---- clip divisor ----
   if (!exact_norm) {  // the update norm in the reference's order (came8_norm.h)
     using EstFn = void (*)(const DevTensor*, const int32_t*, const int64_t*, int, Hp);
@@ -1593,7 +1633,6 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     }
     if ((rc = launch_walk(plan.nwalk, plan.nfinal, stream)) != CAME8_OK) return rc;
   }
-  const bool any2d = !plan.tiles2d.empty() || !plan.tiles2d_v.empty();
   if (exact_norm || any2d) {  // reference order: only the 8bit2d tensors take this divisor
     PhaseTimer pt(PH_CLIP, 0.0, stream);
     hipLaunchKernelGGL(k_clip<>, dim3(grid_for(n_tensors)), blk, 0, stream, dT, int(n_tensors), int(!exact_norm), hp);
@@ -1631,11 +1670,13 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
       if ((rc = check_launch("res_rows2d")) != CAME8_OK) return rc;
     }
     if ((rc = pq.finish()) != CAME8_OK) return rc;
-    const WorkList& fb = plan.factor;
-    { PhaseTimer pt(PH_FACTOR_RES, alg_bytes(plan, fb, tensors, PH_FACTOR_RES), stream);
-    hipLaunchKernelGGL(k_factor_blocks<true>, dim3(grid_for(fb.total())), blk, 0, stream, dT, tids(fb), wst(fb),
-                       int(fb.tids.size()), hp);
-    if ((rc = check_launch("factor_blocks_res")) != CAME8_OK) return rc; }
+    if (any_factor) {
+      const WorkList& fb = plan.factor;
+      PhaseTimer pt(PH_FACTOR_RES, alg_bytes(plan, fb, tensors, PH_FACTOR_RES), stream);
+      launch_factor(k_factor_blocks<true, 4>, k_factor_blocks<true, 8>, fb, factor_lds(4, false), factor_lds(8, false));
+      if ((rc = check_launch("factor_blocks_res")) != CAME8_OK) return rc;
+    }
+    if ((rc = launch_state_quant(k_state_quant<true>, "state_quant_res")) != CAME8_OK) return rc;
   }
   // ---- P3 and 1-D pass B ----
   for (auto& kv : plan.param2d_v) {

@@ -827,111 +827,6 @@ __global__ __launch_bounds__(TPB) void k_fact_pass1n(const DevTensor* __restrict
   }
 }
 
-// ---------------- P1 / P2 for tiny matrices ----------------
-// Tensors whose matrices hold at most kTinyElems elements (conv kernels such as 320x320x3x3 are
-// 102400 matrices of 3x3; 1280x640x1x1 is 819200 matrices of one element) take one thread per
-// matrix instead of a workgroup per band: the matrix is its own band (nbands = 1), and the thread
-// writes what the band passes write -- new row states, the band's row-state sum, the column partial
-// sums -- with the same per-element arithmetic, its sums in fp64 in index order.
-constexpr int kTinyElems = 64;
-
-template <typename TG>
-__global__ __launch_bounds__(kThreads) void k_tiny_pass1(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
-                                                         const int64_t* __restrict__ wstart, int ntens, Hp hp) {
-  using GS = typename TG::storage;
-  const int64_t total = wstart[ntens];
-  for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
-    const int slot = find_slot(wstart, ntens, w);
-    const DevTensor& t = T[tids[slot]];
-    const int64_t b = (w - wstart[slot]) * kThreads + threadIdx.x;  // the matrix
-    if (b >= t.P) continue;
-    const int64_t R = t.R, C = t.C;
-    const CAME8_GLOBAL GS* __restrict__ g = gbl(static_cast<const GS*>(t.g) + b * R * C);
-    CAME8_GLOBAL float* __restrict__ Rn = gbl(t.Rn + b * R);
-    const float invC = 1.0f / float(C);
-    double bandR = 0.0;
-    for (int64_t i = 0; i < R; ++i) {
-      double s = 0.0;
-      for (int64_t j = 0; j < C; ++j) {
-        const double x = double(TG::load(g[i * C + j]));
-        s = fma(x, x, s);
-      }
-      const int64_t row = b * R + i;
-      const float Rold = t.fp32st ? st_sq_row(t)[row] : deq_u8(t.rq[row], t.ra[rblk(t, row, hp)]);
-      const float mean = float(s + double(C) * double(hp.eps0)) * invC;
-      const float Rnew = fmaf(mean, hp.a2, Rold * hp.b2);
-      Rn[i] = Rnew;
-      bandR += Rnew;
-    }
-    const float band_eps = float(R) * hp.eps0;
-    for (int64_t j = 0; j < C; ++j) {
-      double u = 0.0;
-      float wsum = 0.0f;
-      for (int64_t i = 0; i < R; ++i) {
-        const float x = TG::load(g[i * C + j]);
-        u = fma(double(x), double(x), u);
-        wsum = fmaf(x * __builtin_amdgcn_rcpf(Rn[i]), x, wsum);
-      }
-      gbl(t.partU)[b * C + j] = float(u) + band_eps;
-      gbl(t.partW)[b * C + j] = wsum;
-    }
-    gbl(t.rsum)[b] = float(bandR);
-  }
-}
-
-template <typename TG>
-__global__ __launch_bounds__(kThreads) void k_tiny_pass2(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
-                                                         const int64_t* __restrict__ wstart, int ntens, Hp hp) {
-  using GS = typename TG::storage;
-  const int64_t total = wstart[ntens];
-  for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
-    const int slot = find_slot(wstart, ntens, w);
-    const DevTensor& t = T[tids[slot]];
-    const int64_t b = (w - wstart[slot]) * kThreads + threadIdx.x;
-    if (b >= t.P) continue;
-    const int64_t R = t.R, C = t.C, e0 = b * R * C;
-    const CAME8_GLOBAL GS* __restrict__ g = gbl(static_cast<const GS*>(t.g) + e0);
-    const CAME8_GLOBAL float* __restrict__ rf = gbl(t.rfac + b * R);
-    const CAME8_GLOBAL float* __restrict__ cf = gbl(t.cfac + b * C);
-    const float clip = t.clip[0];
-    const float crcp = 1.0f / clip;  // as the band pass: the divisor is >= 1
-    const int64_t PR = t.P * R;
-    // d = u - m of element (i, j), as the band pass forms it
-    auto d_at = [&](int64_t i, int64_t j) {
-      const int64_t e = e0 + i * C + j;
-      const float mo = t.fp32st ? st_m(t)[e]
-                                : float(t.mq[e]) * div_fast(t.ma[t.pm ? mblk(t, e, hp) : blk_of_nb(e, hp)], kSignedQ, kRcpSignedQ);
-      const float u = div_fast((rf[i] * cf[j]) * TG::load(g[i * C + j]), clip, crcp);
-      const float m = fmaf(u, hp.a1, mo * hp.b1);
-      return u - m;
-    };
-    double bandRR = 0.0;
-    for (int64_t i = 0; i < R; ++i) {
-      double s = 0.0;
-      for (int64_t j = 0; j < C; ++j) {
-        const float d = d_at(i, j);
-        s = fma(double(d), double(d), s);
-      }
-      const int64_t row = b * R + i;
-      const float tot = float(s + double(C) * double(hp.eps1));
-      const float RRold = t.fp32st ? t.ra[row] : deq_u8(t.rq[PR + row], t.ra[t.nbr + rblk(t, row, hp)]);
-      const float RRnew = fmaf(tot / float(C), hp.a3, RRold * hp.b3);
-      gbl(t.RRn)[row] = RRnew;
-      bandRR += RRnew;
-    }
-    const float band_eps = float(R) * hp.eps1;
-    for (int64_t j = 0; j < C; ++j) {
-      double s = 0.0;
-      for (int64_t i = 0; i < R; ++i) {
-        const float d = d_at(i, j);
-        s = fma(double(d), double(d), s);
-      }
-      gbl(t.partRes)[b * C + j] = float(s) + band_eps;
-    }
-    gbl(t.rrsum)[b] = float(bandRR);
-  }
-}
-
 // ---------------- P2 ----------------
 // Residual row and column sums of a band.  Per element the reference forms u = (r_i*c_j)*g / clip,
 // m = fma(u, 1-b1, m_old*b1) and res = (u - m)^2 + eps1 (CAME8bitFull.py:1032-1036) and keeps only
@@ -1275,38 +1170,84 @@ __device__ __forceinline__ float matrix_row_mean(const DevTensor& t, const float
   return row_mean_of_sum(t, ordered_sum_f64(bandsum + b * nb, nb, 1));
 }
 
-// Sums over the nbands band partials of one column (stride C) of one or two partial arrays: four
-// interleaved fp64 accumulators (band k into accumulator k % 4), combined as (a0 + a1) + (a2 + a3).
-template <int NA>
-__device__ __forceinline__ void band_column_sums(const float* __restrict__ p0, const float* __restrict__ p1,
-                                                 int64_t nbands, int64_t C, double* out) {
-  double a[NA][4] = {};
-  int64_t k = 0;
-  for (; k + kSumBatch <= nbands; k += kSumBatch) {
-    float v[NA][kSumBatch];
+// A column block's sums over its band partials are spread over the workgroup's NW wavefronts: wavefront w adds
+// bands w, w + NW, ... of 256 columns (four a lane, every load 256 contiguous bytes, a batch of bands in flight), and
+// the wavefronts' fp64 sums are added in order through LDS.  One thread per column waited for nbands / 16 memory
+// round trips.  NW is 4 (every thread finishes a column), or 8 where a launch has too few blocks to occupy the GPU
+// with those (came8.hip; 16 spill).
+constexpr int kFactorCols = 256;
+// LDS of a launch: the wavefronts' sums of one or two partial arrays
+constexpr size_t factor_lds(int nw, bool two_arrays) {
+  return sizeof(double) * nw * kFactorCols * (two_arrays ? 2 : 1);
+}
+
+// row of row state / column of column state i of a tensor, and its matrix
+__device__ __forceinline__ int64_t row_matrix(const DevTensor& t, int64_t i) {
+  return t.idx32 ? int64_t(udiv_magic(uint32_t(i), t.mR, t.sR)) : i / t.R;
+}
+__device__ __forceinline__ int64_t col_matrix(const DevTensor& t, int64_t i) {
+  return t.idx32 ? int64_t(udiv_magic(uint32_t(i), t.mC, t.sC)) : i / t.C;
+}
+
+// This wavefront's share of the band sums of the columns [cb, cb + kFactorCols) (past i1: column i1 - 1 again).
+// ONE: the columns are one matrix's, so a band's row of partials starts at the same address for every lane.
+template <int NA, int NW, bool ONE>
+__device__ __forceinline__ void band_column_part(const DevTensor& t, const float* __restrict__ p0,
+                                                 const float* __restrict__ p1, int64_t cb, int64_t i1, int lane,
+                                                 int wid, double* psum) {
+  constexpr int U = ONE ? 8 / NA : 4;  // bands in flight
+  using Off = typename std::conditional<ONE, uint32_t, int64_t>::type;
+  const int64_t nb = t.nbands, C = t.C;
+  const int64_t b0 = col_matrix(t, cb), base = ONE ? b0 * nb * C : 0;
+  Off off[4];
 #pragma unroll
-    for (int u = 0; u < kSumBatch; ++u) {
-      v[0][u] = p0[(k + u) * C];
-      if constexpr (NA > 1) v[NA - 1][u] = p1[(k + u) * C];
+  for (int q = 0; q < 4; ++q) {
+    const int64_t i = min(cb + q * kWave + lane, i1 - 1);
+    if constexpr (ONE) {
+      off[q] = uint32_t(i - b0 * C);
+    } else {
+      const int64_t b = col_matrix(t, i);
+      off[q] = (b * nb) * C + (i - b * C);
+    }
+  }
+  const CAME8_GLOBAL float* __restrict__ g0 = gbl(p0) + base;
+  const CAME8_GLOBAL float* __restrict__ g1 = NA > 1 ? gbl(p1) + base : g0;
+  double acc[NA][4] = {};
+  for (int64_t k = wid; k < nb; k += NW * U) {
+    float v[NA][U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t o = min(k + u * NW, nb - 1) * C;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        v[0][u][q] = (g0 + o)[off[q]];
+        if constexpr (NA > 1) v[NA - 1][u][q] = (g1 + o)[off[q]];
+      }
     }
 #pragma unroll
-    for (int x = 0; x < NA; ++x)
+    for (int u = 0; u < U; ++u) {
+      const bool in = k + u * NW < nb;  // a band past the last counts for nothing
 #pragma unroll
-      for (int u = 0; u < kSumBatch; ++u) a[x][u & 3] += double(v[x][u]);
-  }
-  for (; k < nbands; ++k) {
-    a[0][0] += double(p0[k * C]);
-    if constexpr (NA > 1) a[NA - 1][0] += double(p1[k * C]);
+      for (int x = 0; x < NA; ++x)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[x][q] += in ? double(v[x][u][q]) : 0.0;
+    }
   }
 #pragma unroll
-  for (int x = 0; x < NA; ++x) out[x] = (a[x][0] + a[x][1]) + (a[x][2] + a[x][3]);
+  for (int x = 0; x < NA; ++x)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) psum[(x * NW + wid) * kFactorCols + q * kWave + lane] = acc[x][q];
 }
-template <bool RES>
-__global__ __launch_bounds__(kThreads) void k_factor_blocks(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
-                                                            const int64_t* __restrict__ wstart, int ntens, Hp hp) {
-  __shared__ float smax[4];
-  __shared__ double ssum[4], msum[4];
+
+template <bool RES, int NW>
+__global__ __launch_bounds__(NW * kWave) void k_factor_blocks(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
+                                                                  const int64_t* __restrict__ wstart, int ntens, Hp hp) {
+  constexpr int NA = RES ? 1 : 2;
+  extern __shared__ double psum[];  // [array][wavefront][column] (factor_lds)
+  __shared__ float smax[NW];
+  __shared__ double ssum[NW], msum[NW];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  constexpr int nt = NW * kWave;
   const int64_t total = wstart[ntens];
   for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
     const int slot = find_slot(wstart, ntens, w);
@@ -1332,29 +1273,32 @@ __global__ __launch_bounds__(kThreads) void k_factor_blocks(const DevTensor* __r
     const float alpha = RES ? hp.a3 : hp.a2;
     const float alpha_f = RES ? hp.a3f : hp.a2f;
     if (is_row) {
-      const float* __restrict__ Rsrc = RES ? t.RRn : t.Rn;
+      const float* Rsrc = RES ? t.RRn : t.Rn;
       float* __restrict__ fac = RES ? t.rrfac : t.rfac;
       const float* __restrict__ bsum = RES ? t.rrsum : t.rsum;
       // the 8bit2d momentum pass sums its residual row states per tile row
       const int64_t nsum = (RES && t.mode2d) ? int64_t(t.tr) : t.nbands;
-      int64_t mb = i0 / t.R;  // matrix of the block's first row; blocks may span matrices
+      int64_t mb = row_matrix(t, i0);  // matrix of the block's first row; blocks may span matrices
       const float vfirst = i0 + tid < i1 ? Rsrc[i0 + tid] : 0.0f;  // loaded before the mean's sums
       float mean;
-      if ((i1 - 1) / t.R == mb) {
+      if (row_matrix(t, i1 - 1) == mb) {
         // the block's rows are one matrix's (uniform): the workgroup sums the matrix's band sums together,
-        // thread k over sums k, k + 256, ..., then in a fixed order (one round of loads instead of one
+        // thread k over sums k, k + nt, ..., then in a fixed order (one round of loads instead of one
         // thread's chain over all of them)
         double ms = 0.0;
-        for (int64_t k = tid; k < nsum; k += kThreads) ms += double(bsum[mb * nsum + k]);
+        for (int64_t k = tid; k < nsum; k += nt) ms += double(bsum[mb * nsum + k]);
         ms = wave_sum(ms);
         if (lane == 0) msum[wid] = ms;
         __syncthreads();  // (msum is written again only after the block maximum's barrier below)
-        mean = row_mean_of_sum(t, ((msum[0] + msum[1]) + msum[2]) + msum[3]);
+        ms = msum[0];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) ms += msum[k];
+        mean = row_mean_of_sum(t, ms);
       } else {
         mean = matrix_row_mean(t, bsum, mb, nsum);
       }
-      for (int64_t i = i0 + tid; i < i1; i += kThreads) {
-        const int64_t bi = i / t.R;
+      for (int64_t i = i0 + tid; i < i1; i += nt) {
+        const int64_t bi = row_matrix(t, i);
         if (bi != mb) {
           mb = bi;
           mean = matrix_row_mean(t, bsum, mb, nsum);
@@ -1368,54 +1312,84 @@ __global__ __launch_bounds__(kThreads) void k_factor_blocks(const DevTensor* __r
       const int64_t off = RES ? t.P * t.C : 0;
       const int64_t aoff = RES ? t.nbc : 0;
       const float* __restrict__ part = RES ? t.partRes : t.partU;
-      float* __restrict__ Cdst = RES ? t.CRn : t.Cn;
+      float* Cdst = RES ? t.CRn : t.Cn;
       float* __restrict__ fac = RES ? t.crfac : t.cfac;
+      float* __restrict__ cst = RES ? t.ca : st_sq_col(t);  // fp32 column state
       const float fR = float(t.R);
+      // column sums of the clip weights too (the default clip mode's band passes wrote no partW)
+      const bool withW = !RES && (t.mode2d || !hp.noW);
       int64_t cmb = -1;  // matrix whose mean row state crm holds
       float crm = 0.0f;
-      for (int64_t i = i0 + tid; i < i1; i += kThreads) {
-        const int64_t b = i / t.C;
-        const int64_t j = i - b * t.C;
-        float* __restrict__ cst = RES ? t.ca : st_sq_col(t);  // fp32 column state
-        float Cold, Cv;
-        double W = 0.0;  // column sum of the clip weights (!RES)
-        if (t.mode2d) {
-          // 8bit2d: residual column sums come from the tile partials (tiles in order); no clamp
-          float s2 = 0.0f;
-          if (RES) {
-            s2 = ordered_sum_f32(t.t2col + i, t.tr, t.C);
-          } else {
-            double sw[2];
-            band_column_sums<2>(part + (b * t.nbands) * t.C + j, t.partW + (b * t.nbands) * t.C + j, t.nbands, t.C, sw);
-            s2 = float(sw[0]);
-            W = sw[1];
+      if (withW && col_matrix(t, i1 - 1) == col_matrix(t, i0)) {  // one matrix's block (uniform): as for a row block
+        cmb = col_matrix(t, i0);
+        double ms = 0.0;
+        for (int64_t k = tid; k < t.nbands; k += nt) ms += double(t.rsum[cmb * t.nbands + k]);
+        ms = wave_sum(ms);
+        if (lane == 0) msum[wid] = ms;
+        __syncthreads();
+        ms = msum[0];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) ms += msum[k];
+        crm = row_mean_of_sum(t, ms);
+      }
+      for (int64_t cb = i0; cb < i1; cb += kFactorCols) {
+        const int64_t i = cb + tid;
+        const bool own = tid < kFactorCols && i < i1;  // this thread finishes column i
+        // the old state's loads go out before the partial sums' (their latencies overlap)
+        float Cold = 0.0f;
+        if (own) {
+          if (t.mode2d) Cold = RES ? deq_u8(t.rcq[i], t.rca[blk_of(i, hp)]) : deq_u8(t.cq[i], t.ca[blk_of(i, hp)]);
+          else Cold = t.fp32st ? cst[i] : deq_u8(t.cq[off + i], t.ca[aoff + cblk(t, i, hp)]);
+        }
+        float s = 0.0f;
+        double W = 0.0;
+        if (RES && t.mode2d) {
+          // 8bit2d: a float32 sum from zero over the tile rows in order (the reference's), 16 loads at a time
+          if (own) s = ordered_sum_f32(t.t2col + i, t.tr, t.C);
+        } else if (t.nbands == 1) {  // one band a matrix (small matrices): its partial is the sum
+          if (own) {
+            s = part[i];
+            if (withW) W = double(t.partW[i]);
           }
-          Cold = RES ? deq_u8(t.rcq[i], t.rca[blk_of(i, hp)]) : deq_u8(t.cq[i], t.ca[blk_of(i, hp)]);
-          Cv = (Cold * beta) + (alpha_f * (s2 / fR));
         } else {
-          const float* __restrict__ pp = part + (b * t.nbands) * t.C + j;
-          // the old state's loads go out before the partial sums' (their latencies overlap)
-          Cold = t.fp32st ? cst[i] : deq_u8(t.cq[off + i], t.ca[aoff + cblk(t, i, hp)]);
-          double sw[2] = {0.0, 0.0};  // column sums of the partials, and for !RES of the clip weights
-          // (in the default clip mode the band passes wrote no partW: the clip partial is not used)
-          if (RES || hp.noW) band_column_sums<1>(pp, nullptr, t.nbands, t.C, sw);
-          else band_column_sums<2>(pp, t.partW + (b * t.nbands) * t.C + j, t.nbands, t.C, sw);
-          const double s = sw[0];
-          W = sw[1];
-          Cv = clamp_min_tiny(fmaf(float(s) / fR, alpha, Cold * beta));
-        }
-        const float c = rsqrt_ref(Cv);
-        Cdst[i] = Cv;
-        fac[i] = c;
-        if (t.fp32st) cst[i] = Cv;
-        vmax = nan_max(vmax, Cv);
-        if (!RES && (t.mode2d || !hp.noW)) {  // the clip partial (k_clip: exact mode, and 8bit2d tensors always)
-          if (b != cmb) {
-            cmb = b;
-            crm = matrix_row_mean(t, t.rsum, b, t.nbands);
+          const bool one = col_matrix(t, min(cb + kFactorCols, i1) - 1) == col_matrix(t, cb);  // uniform
+          if (withW) {
+            if (one) band_column_part<NA, NW, true>(t, part, t.partW, cb, i1, lane, wid, psum);
+            else band_column_part<NA, NW, false>(t, part, t.partW, cb, i1, lane, wid, psum);
+          } else {
+            if (one) band_column_part<1, NW, true>(t, part, nullptr, cb, i1, lane, wid, psum);
+            else band_column_part<1, NW, false>(t, part, nullptr, cb, i1, lane, wid, psum);
           }
-          csum += double(crm) * double(c) * double(c) * W;
+          __syncthreads();
+          if (own) {
+            double a0 = psum[tid], a1 = withW ? psum[(NA - 1) * NW * kFactorCols + tid] : 0.0;
+#pragma unroll
+            for (int k = 1; k < NW; ++k) {
+              a0 += psum[k * kFactorCols + tid];
+              if (withW) a1 += psum[((NA - 1) * NW + k) * kFactorCols + tid];
+            }
+            s = float(a0);
+            W = a1;
+          }
         }
+        if (own) {
+          const float Cv = t.mode2d ? (Cold * beta) + (alpha_f * (s / fR))  // 8bit2d: no clamp
+                                    : clamp_min_tiny(fmaf(s / fR, alpha, Cold * beta));
+          const float c = rsqrt_ref(Cv);
+          Cdst[i] = Cv;
+          fac[i] = c;
+          if (t.fp32st) cst[i] = Cv;
+          vmax = nan_max(vmax, Cv);
+          if (withW) {  // the clip partial (k_clip: exact mode, and 8bit2d tensors always)
+            const int64_t b = col_matrix(t, i);
+            if (b != cmb) {
+              cmb = b;
+              crm = matrix_row_mean(t, t.rsum, b, t.nbands);
+            }
+            csum += double(crm) * double(c) * double(c) * W;
+          }
+        }
+        if (cb + kFactorCols < i1) __syncthreads();  // psum is written again
       }
     }
     // block max and clip partial (fixed order)
@@ -1426,9 +1400,17 @@ __global__ __launch_bounds__(kThreads) void k_factor_blocks(const DevTensor* __r
       ssum[wid] = csum;
     }
     __syncthreads();
-    const float amax = fix_absmax(nan_max(nan_max(smax[0], smax[1]), nan_max(smax[2], smax[3])));
+    vmax = smax[0];
+#pragma unroll
+    for (int k = 1; k < NW; ++k) vmax = nan_max(vmax, smax[k]);
+    const float amax = fix_absmax(vmax);
     if (tid == 0) {
-      if (!RES && !is_row) t.clip_part[blk] = ((ssum[0] + ssum[1]) + ssum[2]) + ssum[3];
+      if (!RES && !is_row) {
+        double cs = ssum[0];
+#pragma unroll
+        for (int k = 1; k < NW; ++k) cs += ssum[k];
+        t.clip_part[blk] = cs;
+      }
       if (t.mode2d) {
         if (is_row) (RES ? t.rra : t.ra)[blk] = amax;
         else (RES ? t.rca : t.ca)[blk] = amax;
@@ -1438,23 +1420,276 @@ __global__ __launch_bounds__(kThreads) void k_factor_blocks(const DevTensor* __r
       }
     }
     const float arcp = rcp_for_div(amax);
-    if (t.fp32st) {
-      // fp32 states were written above; no codes
-    } else if (t.mode2d) {
-      const float inv = 1.0f / amax;
-      const float* __restrict__ src = is_row ? (RES ? t.RRn : t.Rn) : (RES ? t.CRn : t.Cn);
-      uint8_t* __restrict__ q = is_row ? (RES ? t.rrq : t.rq) : (RES ? t.rcq : t.cq);
-      for (int64_t i = i0 + tid; i < i1; i += kThreads) q[i] = quant_u8_inv(src[i], inv);
-    } else if (is_row) {
-      const float* __restrict__ Rsrc = RES ? t.RRn : t.Rn;
-      uint8_t* __restrict__ q = t.rq + (RES ? t.P * t.R : 0);
-      for (int64_t i = i0 + tid; i < i1; i += kThreads) q[i] = quant_u8_r(Rsrc[i], amax, arcp);
-    } else {
-      const float* __restrict__ Csrc = RES ? t.CRn : t.Cn;
-      uint8_t* __restrict__ q = t.cq + (RES ? t.P * t.C : 0);
-      for (int64_t i = i0 + tid; i < i1; i += kThreads) q[i] = quant_u8_r(Csrc[i], amax, arcp);
+    // the codes: each thread those of the states it wrote (a column's thread is one of the first kFactorCols)
+    if (!t.fp32st && (is_row || tid < kFactorCols)) {
+      const float* src = is_row ? (RES ? t.RRn : t.Rn) : (RES ? t.CRn : t.Cn);
+      uint8_t* __restrict__ q;
+      if (t.mode2d) q = is_row ? (RES ? t.rrq : t.rq) : (RES ? t.rcq : t.cq);
+      else q = is_row ? t.rq + (RES ? t.P * t.R : 0) : t.cq + (RES ? t.P * t.C : 0);
+      const float inv = 1.0f / amax;  // 8bit2d
+      const int step = is_row ? nt : kFactorCols;
+      for (int64_t i = i0 + tid; i < i1; i += step) {
+        const float v = src[i];
+        q[i] = t.mode2d ? quant_u8_inv(v, inv) : quant_u8_r(v, amax, arcp);
+      }
     }
     __syncthreads();  // smax / ssum reused by the next item
+  }
+}
+
+// ---------------- P1 / P2 for tiny matrices ----------------
+// Tensors whose matrices hold at most kTinyElems elements (conv kernels such as 320x320x3x3 are
+// 102400 matrices of 3x3; 1280x640x1x1 is 819200 matrices of one element) take one thread per
+// matrix instead of a workgroup per band: the thread has all of its matrix's rows and columns, so it
+// forms the new states and the factors too (the band passes leave those to the factor kernels), with the
+// same per-element arithmetic, its sums in fp64 in index order.  Only the states' requantisation, whose
+// blocks span matrices, follows in k_state_quant.  Pass 1 also sums its matrices' u^2 for the clip: the
+// partial of the exact clip and the unit of the reference-order norm's estimates.
+//
+// A matrix's elements are a few bytes apart from the next one's, so a thread's own loads would touch a line
+// per lane: the workgroup stages its kThreads matrices in LDS with 16-byte loads instead (rows of an odd
+// number of words: bank conflicts) and each thread reads its own there.  22.9 M elements of 3x3 and 1x1
+// matrices, bf16: the two passes and the states' codes 112 + 148 + 59 us; with a thread's own loads, the factor
+// kernels and an estimate kernel it was 86 + 139 + 451 + 532 us.
+constexpr int kTinyElems = 64;
+
+// matrices staged at a time (at most 63 KB of LDS), words between them there, and n / rc for n < 2^14 and
+// rc <= 64 (exact: n * 64 < 2^20)
+constexpr int tiny_batch(int64_t rc) { return rc <= 48 ? kThreads : kThreads / 2; }
+__device__ __forceinline__ int tiny_stride(int rc) { return rc | 1; }
+__device__ __forceinline__ uint32_t tiny_magic(int rc) { return (1u << 20) / uint32_t(rc) + 1u; }
+
+// Stages the elements of matrices [b0, b0 + cnt) (rc each) as floats.  b0 is a multiple of 128, so its first
+// element is 16-byte aligned when the gradient is.  Synchronises.
+template <typename TG>
+__device__ __forceinline__ void tiny_stage_g(const DevTensor& t, int64_t b0, int cnt, int rc, float* lds) {
+  using GS = typename TG::storage;
+  constexpr int V = 16 / int(sizeof(GS));
+  const CAME8_GLOBAL GS* __restrict__ g = gbl(static_cast<const GS*>(t.g) + b0 * rc);
+  const int n = cnt * rc, tid = threadIdx.x;
+  const uint32_t mg = tiny_magic(rc);
+  const bool pad = (rc & 1) == 0;
+  const int nv = (reinterpret_cast<uintptr_t>(t.g) & 15) == 0 ? n / V : 0;
+  for (int i = tid; i < nv; i += kThreads) {
+    const u32x4 r = ld_nt((const CAME8_GLOBAL u32x4*)g + i);
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const uint32_t e = uint32_t(i * V + v);
+      lds[pad ? e + ((e * mg) >> 20) : e] = TG::elem(w, v);
+    }
+  }
+  for (int i = nv * V + tid; i < n; i += kThreads) {
+    const uint32_t e = uint32_t(i);
+    lds[pad ? e + ((e * mg) >> 20) : e] = TG::load(g[i]);
+  }
+  __syncthreads();
+}
+
+// LDS bytes of a launch whose largest matrices hold rc elements (pass 2 stages the momentum codes behind the
+// gradients)
+constexpr size_t tiny_lds(int64_t rc, bool codes) {
+  return size_t(tiny_batch(rc)) * (size_t(rc | 1) * 4 + (codes ? size_t(rc) : 0));
+}
+
+template <typename TG>
+__global__ __launch_bounds__(kThreads) void k_tiny_pass1(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
+                                                         const int64_t* __restrict__ wstart, int ntens, Hp hp) {
+  extern __shared__ float tiny_g[];
+  __shared__ double ssum[4];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int64_t total = wstart[ntens];
+  for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
+    const int slot = find_slot(wstart, ntens, w);
+    const DevTensor& t = T[tids[slot]];
+    const int64_t item = w - wstart[slot];
+    const int R = int(t.R), C = int(t.C), rc = R * C;
+    double usum = 0.0;
+    const int batch = tiny_batch(rc);
+    for (int64_t b0 = item * t.ngrp; b0 < min(t.P, (item + 1) * t.ngrp); b0 += batch) {  // an item: ngrp matrices
+      const int cnt = int(min(int64_t(batch), t.P - b0));
+      tiny_stage_g<TG>(t, b0, cnt, rc, tiny_g);
+      if (tid < cnt) {
+        const int64_t b = b0 + tid;
+        const float* x = tiny_g + tid * tiny_stride(rc);
+        CAME8_GLOBAL float* Rn = gbl(t.Rn + b * R);
+        const float invC = 1.0f / float(C);
+        double bandR = 0.0;
+        for (int i = 0; i < R; ++i) {
+          double s = 0.0;
+          for (int j = 0; j < C; ++j) s = fma(double(x[i * C + j]), double(x[i * C + j]), s);
+          const int64_t row = b * R + i;
+          const float Rold = t.fp32st ? st_sq_row(t)[row] : deq_u8(t.rq[row], t.ra[rblk(t, row, hp)]);
+          const float mean = float(s + double(C) * double(hp.eps0)) * invC;
+          const float Rnew = fmaf(mean, hp.a2, Rold * hp.b2);
+          Rn[i] = Rnew;
+          bandR += Rnew;
+          if (t.fp32st) gbl(st_sq_row(t))[row] = Rnew;
+        }
+        const float rm = row_mean_of_sum(t, double(float(bandR)));
+        CAME8_GLOBAL float* rf = gbl(t.rfac + b * R);
+        for (int i = 0; i < R; ++i) rf[i] = rsqrt_ref(Rn[i] / rm);
+        const float band_eps = float(R) * hp.eps0, fR = float(R);
+        for (int j = 0; j < C; ++j) {
+          double u = 0.0;
+          for (int i = 0; i < R; ++i) u = fma(double(x[i * C + j]), double(x[i * C + j]), u);
+          const int64_t col = b * C + j;
+          const float Cold = t.fp32st ? st_sq_col(t)[col] : deq_u8(t.cq[col], t.ca[cblk(t, col, hp)]);
+          const float Cv = clamp_min_tiny(fmaf((float(u) + band_eps) / fR, hp.a2, Cold * hp.b2));
+          const float c = rsqrt_ref(Cv);
+          gbl(t.Cn)[col] = Cv;
+          gbl(t.cfac)[col] = c;
+          if (t.fp32st) gbl(st_sq_col(t))[col] = Cv;
+          for (int i = 0; i < R; ++i) {
+            const float uu = (rf[i] * c) * x[i * C + j];
+            usum = fma(double(uu), double(uu), usum);
+          }
+        }
+      }
+      __syncthreads();  // the LDS is staged again
+    }
+    usum = wave_sum(usum);
+    if (lane == 0) ssum[wid] = usum;
+    __syncthreads();
+    if (tid == 0) {
+      const double s = ((ssum[0] + ssum[1]) + ssum[2]) + ssum[3];
+      t.clip_part[item] = s;
+      t.nest[item] = float(s);
+    }
+    __syncthreads();
+  }
+}
+
+template <typename TG>
+__global__ __launch_bounds__(kThreads) void k_tiny_pass2(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
+                                                         const int64_t* __restrict__ wstart, int ntens, Hp hp) {
+  extern __shared__ float tiny_g[];
+  const int tid = threadIdx.x;
+  const int64_t total = wstart[ntens];
+  for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
+    const int slot = find_slot(wstart, ntens, w);
+    const DevTensor& t = T[tids[slot]];
+    const int64_t item = w - wstart[slot];
+    const int R = int(t.R), C = int(t.C), rc = R * C;
+    const float clip = t.clip[0];
+    const float crcp = 1.0f / clip;  // as the band pass: the divisor is >= 1
+    const int64_t PR = t.P * R, PC = t.P * C;
+    const int batch = tiny_batch(rc);
+    int8_t* codes = reinterpret_cast<int8_t*>(tiny_g + batch * tiny_stride(rc));
+    for (int64_t b0 = item * t.ngrp; b0 < min(t.P, (item + 1) * t.ngrp); b0 += batch) {
+      const int cnt = int(min(int64_t(batch), t.P - b0));
+      if (!t.fp32st) {  // the matrices' codes, 4 bytes a load where they are aligned
+        const CAME8_GLOBAL int8_t* mq = gbl(t.mq + b0 * rc);
+        const int n = cnt * rc, nv = (reinterpret_cast<uintptr_t>(t.mq) & 3) == 0 ? n / 4 : 0;
+        for (int i = tid; i < nv; i += kThreads)
+          reinterpret_cast<uint32_t*>(codes)[i] = ((const CAME8_GLOBAL uint32_t*)mq)[i];
+        for (int i = nv * 4 + tid; i < n; i += kThreads) codes[i] = mq[i];
+      }
+      tiny_stage_g<TG>(t, b0, cnt, rc, tiny_g);
+      if (tid < cnt) {
+        const int64_t b = b0 + tid, e0 = b * rc;
+        float* x = tiny_g + tid * tiny_stride(rc);
+        const CAME8_GLOBAL float* __restrict__ rf = gbl(t.rfac + b * R);
+        const CAME8_GLOBAL float* __restrict__ cf = gbl(t.cfac + b * C);
+        // d = u - m of every element in its gradient's place, and the row sums of d^2
+        CAME8_GLOBAL float* RRn = gbl(t.RRn + b * R);
+        double bandRR = 0.0;
+        int64_t mb = -1;  // the momentum block of scale sc
+        float sc = 0.0f;
+        for (int i = 0; i < R; ++i) {
+          double s = 0.0;
+          for (int j = 0; j < C; ++j) {
+            const int k = i * C + j;
+            float mo;
+            if (t.fp32st) {
+              mo = st_m(t)[e0 + k];
+            } else {
+              const int64_t eb = t.pm ? mblk(t, e0 + k, hp) : blk_of_nb(e0 + k, hp);
+              if (eb != mb) {
+                mb = eb;
+                sc = div_fast(gbl(t.ma)[eb], kSignedQ, kRcpSignedQ);
+              }
+              mo = float(codes[tid * rc + k]) * sc;
+            }
+            const float u = div_fast((rf[i] * cf[j]) * x[k], clip, crcp);
+            const float d = u - fmaf(u, hp.a1, mo * hp.b1);
+            x[k] = d;
+            s = fma(double(d), double(d), s);
+          }
+          const int64_t row = b * R + i;
+          const float tot = float(s + double(C) * double(hp.eps1));
+          const float RRold = t.fp32st ? t.ra[row] : deq_u8(t.rq[PR + row], t.ra[t.nbr + rblk(t, row, hp)]);
+          const float RRnew = fmaf(tot / float(C), hp.a3, RRold * hp.b3);
+          RRn[i] = RRnew;
+          bandRR += RRnew;
+          if (t.fp32st) gbl(t.ra)[row] = RRnew;
+        }
+        const float rm = row_mean_of_sum(t, double(float(bandRR)));
+        for (int i = 0; i < R; ++i) gbl(t.rrfac)[b * R + i] = rsqrt_ref(RRn[i] / rm);
+        const float band_eps = float(R) * hp.eps1, fR = float(R);
+        for (int j = 0; j < C; ++j) {
+          double s = 0.0;
+          for (int i = 0; i < R; ++i) s = fma(double(x[i * C + j]), double(x[i * C + j]), s);
+          const int64_t col = b * C + j;
+          const float Cold = t.fp32st ? t.ca[col] : deq_u8(t.cq[PC + col], t.ca[t.nbc + cblk(t, col, hp)]);
+          const float Cv = clamp_min_tiny(fmaf((float(s) + band_eps) / fR, hp.a3, Cold * hp.b3));
+          gbl(t.CRn)[col] = Cv;
+          gbl(t.crfac)[col] = rsqrt_ref(Cv);
+          if (t.fp32st) gbl(t.ca)[col] = Cv;
+        }
+      }
+      __syncthreads();  // the LDS is staged again
+    }
+  }
+}
+
+// Codes of the row and column states that the tiny passes formed (RES: the residual ones): a wavefront per
+// state block, four blocks a work item.
+template <bool RES>
+__global__ __launch_bounds__(kThreads) void k_state_quant(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
+                                                          const int64_t* __restrict__ wstart, int ntens, Hp hp) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int64_t total = wstart[ntens];
+  for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
+    const int slot = find_slot(wstart, ntens, w);
+    const DevTensor& t = T[tids[slot]];
+    const int64_t local = (w - wstart[slot]) * 4 + wid;
+    if (local >= t.nbr + t.nbc) continue;  // uniform over the wavefront; no barrier below
+    const bool is_row = local < t.nbr;
+    const int64_t blk = is_row ? local : local - t.nbr;
+    const int64_t n = is_row ? t.R : t.C, len = t.P * n;
+    int64_t i0, i1;
+    if (t.pm) {  // blocks restart at every matrix
+      const int64_t per = is_row ? t.pmb_r : t.pmb_c, mb = blk / per, jb = blk - mb * per;
+      i0 = mb * n + jb * hp.B;
+      i1 = min(i0 + hp.B, (mb + 1) * n);
+    } else {
+      i0 = blk * hp.B;
+      i1 = min(i0 + hp.B, len);
+    }
+    const CAME8_GLOBAL float* __restrict__ src = gbl(static_cast<const float*>(is_row ? (RES ? t.RRn : t.Rn) : (RES ? t.CRn : t.Cn)));
+    CAME8_GLOBAL uint8_t* __restrict__ q = gbl((is_row ? t.rq : t.cq) + (RES ? len : 0));
+    constexpr int kHeld = 4;  // states a lane holds (blocks of 256); later ones are read again
+    float v[kHeld];
+    float vmax = (i1 - i0) < hp.B ? 0.0f : -__builtin_inff();  // zero padding joins the max
+#pragma unroll
+    for (int k = 0; k < kHeld; ++k) {
+      const int64_t i = i0 + lane + k * kWave;
+      v[k] = src[min(i, i1 - 1)];  // past the end: the last state again
+      vmax = nan_max(vmax, v[k]);
+    }
+    for (int64_t i = i0 + lane + kHeld * kWave; i < i1; i += kWave) vmax = nan_max(vmax, src[i]);
+    const float amax = fix_absmax(group_max<64>(vmax)), arcp = rcp_for_div(amax);
+    if (lane == 0) {
+      if (is_row) t.ra[(RES ? t.nbr : 0) + blk] = amax;
+      else t.ca[(RES ? t.nbc : 0) + blk] = amax;
+    }
+#pragma unroll
+    for (int k = 0; k < kHeld; ++k) {
+      const int64_t i = i0 + lane + k * kWave;
+      if (i < i1) q[i] = quant_u8_r(v[k], amax, arcp);
+    }
+    for (int64_t i = i0 + lane + kHeld * kWave; i < i1; i += kWave) q[i] = quant_u8_r(src[i], amax, arcp);
   }
 }
 
@@ -1785,6 +2020,45 @@ __global__ __launch_bounds__(kThreads) void k_fact_pass3(const DevTensor* __rest
         continue;
       }
 
+      uint32_t abits = 0;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) abits = max(abits, abs_bits(m[v]));
+      abits = block_max_bits(abits, L, wmax, par);
+      const float amax = fix_absmax(__uint_as_float(abits));
+      if ((e0 & (hp.B - 1)) == 0) ma[blk] = amax;
+      st_nt((CAME8_GLOBAL u32x2*)(mq + e0), p3_quant8(m, amax, abits));
+    } else if (t.vec_ok && base + kTile <= N) {
+      // ---- rows of fewer than 8 elements (conv kernels): the same vector access, each element's factors gathered
+      // by its row and column (22.9 M elements of 3x3 and 1x1 matrices, bf16: 97 us, 167 element by element) ----
+      float gv[8], pv[8], q[8], m[8], ri[8], rri[8], cj[8], crj[8];
+      load8<TG, true>(g + e0, gv);
+      load8<TP, true>(p + e0, pv);
+      if constexpr (F32ST) load8<F32, true>(gbl(st_m(t)) + e0, q);
+      else load_codes<8>(mq + e0, q);
+      const float amax_old = F32ST ? 0.0f : ma[blk];
+      int64_t cb = bb * C;  // the matrix's first column factor
+      int32_t jj = int32_t(j), left = int32_t(R - 1 - (row - bb * R)), dr = 0;  // rows left in the matrix
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        ri[v] = rfac[row + dr];
+        rri[v] = rrfac[row + dr];
+        cj[v] = cfac[cb + jj];
+        crj[v] = crfac[cb + jj];
+        if (++jj == int32_t(C)) {
+          jj = 0;
+          ++dr;
+          if (--left < 0) {
+            left = int32_t(R) - 1;
+            cb += C;
+          }
+        }
+      }
+      p3_math8r<TP, F32ST>(gv, q, pv, m, amax_old, ri, rri, cj, crj, clip, crcp, clip_fast, hp);
+      store8<TP>(p + e0, pv);
+      if constexpr (F32ST) {
+        store8<F32>(gbl(st_m(t)) + e0, m);
+        continue;
+      }
       uint32_t abits = 0;
 #pragma unroll
       for (int v = 0; v < 8; ++v) abits = max(abits, abs_bits(m[v]));

@@ -143,8 +143,8 @@ constexpr uint32_t kNormFull = 1u << 24;
 // ---------------------------------------------------------------------------
 // Units: row band b of matrix m (unit m * nbands + b; for matrices of the thread-per-matrix passes the
 // matrix is its band) or 2048-element tile u of a 1-D tensor.  The sum of u_ij^2 over a band is
-// rm * sum_i (1 / R_i) * sum_j c_j^2 * g_ij^2 without the roundings.  A matrix of the thread-per-matrix
-// passes has it from W_j = sum_i g_ij^2 / R_i (their column partials): rm * sum_j c_j^2 * W_j.  The band
+// rm * sum_i (1 / R_i) * sum_j c_j^2 * g_ij^2 without the roundings.  The thread-per-matrix passes form u
+// themselves and write their groups' sums of u^2 (k_tiny_pass1).  The band
 // passes of the default clip mode keep no W (k_fact_pass1n); their estimate gives every row of the band
 // the band's column profile of g^2 (the partials U_j):
 //   rm * (sum_i e_i / R_i) * (sum_j c_j^2 U_j) / (sum_j U_j),   e_i = sum_j g_ij^2,
@@ -225,14 +225,7 @@ __global__ __launch_bounds__(kThreads) void k_norm_est(const DevTensor* __restri
       const int64_t b0 = u * t.ngrp, b1 = min(nbase, b0 + t.ngrp);
       float e = 0.0f;
       for (int64_t b = b0; b < b1; ++b) {
-        if (t.factored && t.R * t.C <= kTinyElems) {  // the thread-per-matrix passes wrote W
-          const int64_t m = b / t.nbands;
-          const float* __restrict__ W = t.partW + b * t.C;
-          const float* __restrict__ cf = t.cfac + m * t.C;
-          float s = 0.0f;
-          for (int64_t j = 0; j < t.C; ++j) s = fmaf(cf[j] * cf[j], W[j], s);
-          e += norm_unit_rm(t, b) * s;
-        } else if (t.factored) {  // a band pass of the default mode: the band's profile of g^2
+        if (t.factored) {  // a band pass of the default mode: the band's profile of g^2
           const int64_t m = b / t.nbands;
           const float* __restrict__ Up = t.partU + b * t.C;
           const float* __restrict__ cf = t.cfac + m * t.C;
