@@ -595,6 +595,17 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
       }
   }
 
+  // few record-rebuild work items: halve them (kNormFixMinSegs)
+  {
+    int64_t nfseg = kNormFixSegs;
+    for (; nfseg > kNormFixMinSegs; nfseg >>= 1) {
+      int64_t items = 0;
+      for (const DevTensor& d : plan.dev) items += d.nseg > 1 ? ceil_div(d.nseg, nfseg) : 0;
+      if (items >= kNormFixMinItems) break;
+    }
+    for (DevTensor& d : plan.dev) d.nfseg = nfseg;
+  }
+
   // --- work lists ---
   const bool fastB = fast_block(B);
   // The long-chain group: factored tensors with more than half the longest chain's segments, when the
@@ -687,7 +698,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
         add_item(plan.nseg2d[t.grad_dtype * 3 + (d.c8 ? kNormVec : kNormRows)], i, ceil_div(d.nseg0, d.nrun));
       if (d.nseg > d.nseg0) add_item(plan.nseg[t.grad_dtype * 3 + form], i, d.nseg - d.nseg0);
       if (d.nblk > kNormFixDirect) add_item(plan.nbsum, i, d.nblk);
-      add_item(plan.nfix[t.grad_dtype * 3 + form], i, ceil_div(d.nseg, int64_t(kNormFixSegs)));
+      add_item(plan.nfix[t.grad_dtype * 3 + form], i, ceil_div(d.nseg, d.nfseg));
     }
     add_item((longc[i] ? plan.nwalkL : plan.nwalk)[t.grad_dtype], i, 8);
     add_item((longc[i] ? plan.nfinalL : plan.nfinal)[t.grad_dtype], i, 1);

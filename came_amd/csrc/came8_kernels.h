@@ -75,6 +75,7 @@ struct alignas(128) DevTensor {  // each descriptor on whole cache lines
   float* nsum;        // per chain and segment: fp32 sum of the rounded squares      [8][nseg]
   float* nbsum;       // their sums per block of 256 segments                        [8][nblk]
   int64_t nblk;
+  int64_t nfseg;      // segments per work item of k_norm_fix
   float* nchain;      // the eight chain accumulators                           [8]
   uint64_t mC, mR;    // magic multipliers for n / C and n / R (n < 2^31)
   uint32_t sC, sR;    // and their shifts

@@ -936,7 +936,12 @@ __device__ __forceinline__ void norm_stage_cols(const DevTensor& t, float* cl) {
 // ---------------------------------------------------------------------------
 // each chain's own estimate, and records rebuilt under it
 // ---------------------------------------------------------------------------
-constexpr int kNormFixSegs = kThreads;  // segments per block of the chains' estimates and per work item of k_norm_fix
+constexpr int kNormFixSegs = kThreads;  // segments per block of the chains' estimates, and at most per work item of k_norm_fix
+// Segments whose records need rebuilding come in runs (where the tensor-wide estimate passes a binade boundary), and a
+// work item rebuilds its own, so a launch of few items had one workgroup do hundreds: items are halved, down to
+// kNormFixMinSegs segments, until the launch has kNormFixMinItems (came8.hip).  22.9 M elements of 3x3 and 1x1
+// matrices: 721 us in items of 256 segments, 67 in items of 16; heavy-tailed ragged matrices 410 + 390 -> 81 + 63 us.
+constexpr int64_t kNormFixMinSegs = 16, kNormFixMinItems = 1024;
 constexpr int64_t kNormFixDirect = 4;   // tensors of at most this many blocks: k_norm_fix adds the segments' sums itself
 
 // Each chain's sum of squares over a block of kNormFixSegs segments (nbsum[c][block]), for the prefix
@@ -964,38 +969,40 @@ __global__ __launch_bounds__(kThreads) void k_norm_bsum(const DevTensor* __restr
   }
 }
 
-// The chains' estimates at the segments of one work item of k_norm_fix, into est[c][thread]: the sums of
-// the blocks before it (k_norm_bsum) plus an exclusive scan of the item's own segment sums.
-__device__ __forceinline__ void norm_item_estimates(const DevTensor& t, int64_t blk, const float (&v)[8],
+// The chains' estimates at the segments [base, base + fseg) of one work item of k_norm_fix, into est[c][thread]: the
+// sums of the segments before it plus an exclusive scan of the item's own (v: thread i's segment's, 0 past the item).
+__device__ __forceinline__ void norm_item_estimates(const DevTensor& t, int64_t base, const float (&v)[8],
                                                     float (&est)[8][kNormFixSegs], float (&part)[kThreads / kWave][8],
-                                                    float (&base)[8]) {
+                                                    float (&base_l)[8]) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  // the blocks before this one: thread i adds chain i % 8's blocks i / 8, i / 8 + 32, ... in that order,
-  // four loads in flight at a time.  A tensor of at most kNormFixDirect blocks has no block sums
-  // (k_norm_bsum skips it): its threads add the segments' sums themselves.
+  // thread i adds chain i % 8's sums i / 8, i / 8 + 32, ... in that order, four loads in flight at a time: the whole
+  // blocks before the item (k_norm_bsum; a tensor of at most kNormFixDirect blocks has none) and then the segments
+  // left before it.
   {
     float acc = 0.0f;
     const int c = tid & 7;
     constexpr int kStep = kThreads / 8;
-    const bool direct = t.nblk <= kNormFixDirect;  // uniform
-    const float* __restrict__ nb = direct ? t.nsum + c * t.nseg : t.nbsum + c * t.nblk;
-    const int64_t nend = direct ? blk * kNormFixSegs : blk;
-    int64_t b = tid >> 3;
-    for (; b + 3 * kStep < nend; b += 4 * kStep) {
-      float y[4];
+    auto add = [&](const float* __restrict__ nb, int64_t nend) __attribute__((always_inline)) {
+      int64_t b = tid >> 3;
+      for (; b + 3 * kStep < nend; b += 4 * kStep) {
+        float y[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) y[u] = nb[b + u * kStep];
+        for (int u = 0; u < 4; ++u) y[u] = nb[b + u * kStep];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) acc += y[u];
-    }
-    for (; b < nend; b += kStep) acc += nb[b];
+        for (int u = 0; u < 4; ++u) acc += y[u];
+      }
+      for (; b < nend; b += kStep) acc += nb[b];
+    };
+    const int64_t nblk = t.nblk <= kNormFixDirect ? 0 : base / kNormFixSegs;  // uniform
+    add(t.nbsum + c * t.nblk, nblk);
+    add(t.nsum + c * t.nseg + nblk * kNormFixSegs, base - nblk * kNormFixSegs);
     est[c][tid >> 3] = acc;  // scratch: 32 partials per chain
   }
   __syncthreads();
   if (tid < 8) {
     float acc = 0.0f;
     for (int k = 0; k < kThreads / 8; ++k) acc += est[tid][k];
-    base[tid] = acc;
+    base_l[tid] = acc;
   }
   __syncthreads();
   // this item's segments (v: this thread's segment's sums of squares, 0 past the tensor's segments):
@@ -1018,7 +1025,7 @@ __device__ __forceinline__ void norm_item_estimates(const DevTensor& t, int64_t 
   __syncthreads();
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
-    float off = base[c];
+    float off = base_l[c];
     for (int k = 0; k < kThreads / kWave; ++k) off += k < wid ? part[k][c] : 0.0f;
     est[c][tid] = off + (incl[c] - v[c]);
   }
@@ -1052,7 +1059,7 @@ __device__ __forceinline__ void norm_write_records_pc(const DevTensor& t, int64_
   }
 }
 
-// Records rebuilt under each chain's own estimate.  A work item is kNormFixSegs consecutive segments
+// Records rebuilt under each chain's own estimate.  A work item is t.nfseg consecutive segments
 // of one tensor, one per thread: the chains' estimates at each segment (norm_item_estimates, taken as
 // within [-2%, +0.5%] of the chain) are checked against the segment's eight records, and the segments
 // where a record's binades do not cover a chain's are listed in LDS and shared out to the wavefronts,
@@ -1076,26 +1083,25 @@ __global__ __launch_bounds__(kThreads) void k_norm_fix(const DevTensor* __restri
     const int32_t ti = tids[slot];
     const DevTensor& t = T[ti];
     const int64_t nseg = t.nseg;
-    const int64_t blk = w - wstart[slot];
-    const int64_t base = blk * kNormFixSegs;
-    const int64_t seg = base + tid;
+    const int64_t base = (w - wstart[slot]) * t.nfseg;
+    const int64_t seg = base + tid, end = min(nseg, base + t.nfseg);  // of this item
     if (tid == 0) nlist = 0;
     // this thread's segment's sums of squares and record words, loaded before the estimates' sums
     float v[8];
     uint32_t w0s[8];
     {
-      const int64_t sc = seg < nseg ? seg : nseg - 1;  // nseg >= 1 for a tensor in the list
+      const int64_t sc = seg < end ? seg : end - 1;
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         v[c] = t.nsum[c * nseg + sc];
         w0s[c] = t.nrec[c * nseg + sc];
       }
 #pragma unroll
-      for (int c = 0; c < 8; ++c) v[c] = seg < nseg ? v[c] : 0.0f;
+      for (int c = 0; c < 8; ++c) v[c] = seg < end ? v[c] : 0.0f;
     }
-    norm_item_estimates(t, blk, v, est_l, part, base_l);  // synchronises the workgroup
+    norm_item_estimates(t, base, v, est_l, part, base_l);  // synchronises the workgroup
     uint32_t need = 0;
-    if (seg < nseg) {
+    if (seg < end) {
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         const float est = est_l[c][tid];
