@@ -93,44 +93,29 @@ __device__ __forceinline__ int norm_est_binade(float v) {
   return norm_binade(v);
 }
 
-// The increment of one element whose rounded square is hi under binade E (k = 23 - E) is rint(hi * 2^k),
-// exact for the chain whenever that scaled square dh is not a half-integer and below 2^23 (then
-// half-integers lie on hi's grid, and a true square that is not one rounds like hi).  The segment
-// kernel keeps, per lane and chain, the running sum of rint(dh) and either the largest |dh - rint(dh)|
-// or (k_norm_seg2d) per chain a wavefront mask of the lanes that met a tie (a compare into a scalar
-// register and a scalar or: one VALU instruction per element instead of two); the exceptions are then
-// read off per lane once:
-//   * a tie (some |dh - rint(dh)| = 0.5): the rounding of that element depends on the chain's parity;
-//   * dh >= 2^23: in a normal binade (m >= 2^23) it takes the chain out of the binade by itself, so
-//     the segment's sum, at least 2^23, already fails the walk's test m + sum < 2^24;
-//   * the subnormal binade (E = -126, k = 149), where hi's own rounding may hide a tie: any nonzero
-//     increment there, and any |x| = 2^-75 (NormAcc's TINY form);
-//   * NaN or infinite squares: a NaN or infinite sum.
-// An exception saturates the segment's sum at kNormFull, which makes the walk replay the segment.
-constexpr float kNormSpecial = 0x1p24f;
-__device__ __forceinline__ void norm_acc(float hi, int k, float& sum, float& rmax) {
-  const float dh = ldexpf(hi, k);
-  const float nf = rintf(dh);
-  sum += nf;
-  rmax = fmaxf(rmax, fabsf(dh - nf));
+// The increments of a run of elements under binade E, per lane and chain, without knowing the chain's value: two
+// running sums started inside the binade, at 2^E (even mantissa) and one unit 2^(E-23) above it (odd), each element
+// one fused multiply-add into both.  A fused multiply-add that stays in the binade adds the element's increment,
+// rounded as the chain would round it, so the first sum less its start is the increments' integer sum, exactly; the
+// two sums stay one unit apart unless an element is a tie, which rounds to the even side: then they come out two
+// units or none apart and stay so.  Read off once per lane (norm_lane_value), an exception makes the walk replay
+// the segment:
+//   * a tie: the rounding of that element depends on the chain's parity;
+//   * a sum that left the binade (it only grows; so does one that met a NaN or an infinity): the increments reach
+//     2^23 units, and a chain of a normal binade, whose mantissa is at least 2^23, leaves it too (in the subnormal
+//     binade the replay decides).
+// Squares are exact inside the multiply-add, so the subnormal binade needs no rule of its own.  Five instructions an
+// element with the conversion aside (three products of u, the sum of squares, the two sums; two more per further
+// binade); scaling, rounding and comparing each square took nine, and five more, and bound the records kernel by
+// issue rate (1.07 G bf16 elements: 446 -> 395 us, 5.5 TB/s; one 2048x2048 fp32 matrix: 20.2 -> 13.6 us).
+__device__ __forceinline__ float norm_base(int E) { return __uint_as_float(uint32_t(E + 127) << 23); }
+// the lane's increments for one chain under E as the record's integer, or kNormFull for an exception (E = 128, the
+// binade above the largest, holds no chain)
+__device__ __forceinline__ uint32_t norm_lane_value(float even, float odd, int E) {
+  const uint32_t base = uint32_t(E + 127) << 23;
+  const uint32_t n = __float_as_uint(even) - base;
+  return (n < (1u << 23) && __float_as_uint(odd) - base == n + 1u && E < 128) ? n : (1u << 24);
 }
-// the same, returning whether the element is a tie
-__device__ __forceinline__ bool norm_acc_tie(float hi, int k, float& sum) {
-  const float dh = ldexpf(hi, k);
-  const float nf = rintf(dh);
-  sum += nf;
-  return fabsf(dh - nf) == 0.5f;
-}
-// the lane's sum for one chain as the record's integer, or kNormFull for an exception
-__device__ __forceinline__ uint32_t norm_lane_value(float sum, bool tie, int E) {
-  const bool bad = !(sum < kNormSpecial) || tie || (E == -126 && sum != 0.0f);
-  return bad ? (1u << 24) : uint32_t(sum);
-}
-__device__ __forceinline__ uint32_t norm_lane_value(float sum, float rmax, int E) {
-  return norm_lane_value(sum, rmax == 0.5f, E);
-}
-// lane `lane`'s bit of a wavefront mask
-__device__ __forceinline__ bool norm_bit(uint64_t mask, int lane) { return ((mask >> lane) & 1u) != 0; }
 
 // Record word 0: Ea + 256 (9 bits) | kRecTwo when word 2 holds the sum under Ea + 1.  Words 1 and 2:
 // the integer sums of the increments under Ea and Ea + 1, at most 2^24 (2^24: the segment leaves
@@ -428,71 +413,44 @@ __device__ __forceinline__ void norm_chunk_rows(const DevTensor& t, uint32_t f, 
 // aligned, N < 2^31; the host checks), kNormAny (u_at of each element) for the rest.
 constexpr int kNormAny = 0, kNormRows = 1, kNormVec = 2;
 
-// Per-lane, per-chain accumulators of one segment: the integer sums of the increments under the
-// candidate binades Ea (sa) and Ea + 1 (sb), their largest rounding distances (ra, rb), and the fp32
-// sum of the rounded squares (hs).
+// Per-lane, per-chain accumulators of one segment: the pair of sums under the candidate binade Ea (ae, ao) and
+// under Ea + 1 (be, bo), and the fp32 sum of the squares (hs).
 struct NormAcc {
-  float sa[8], ra[8], sb[8], rb[8], hs[8];
-  __device__ __forceinline__ void clear() {
+  float ae[8], ao[8], be[8], bo[8], hs[8];
+  __device__ __forceinline__ void init(int v, int Ea) {
+    ae[v] = norm_base(Ea);
+    ao[v] = __uint_as_float(__float_as_uint(ae[v]) + 1u);
+    be[v] = norm_base(Ea + 1);
+    bo[v] = __uint_as_float(__float_as_uint(be[v]) + 1u);
+    hs[v] = 0.0f;
+  }
+  __device__ __forceinline__ void init(int Ea) {
 #pragma unroll
-    for (int v = 0; v < 8; ++v) sa[v] = ra[v] = sb[v] = rb[v] = hs[v] = 0.0f;
+    for (int v = 0; v < 8; ++v) init(v, Ea);
   }
-  // element x of chain v under ka = 23 - Ea (TWO: and ka - 1).  TINY: Ea = -126, where |x| = 2^-75
-  // is a tie that x * x hides.
-  template <bool TWO, bool TINY>
-  __device__ __forceinline__ void add(int v, float x, int ka) {
-    const float hi = x * x;
-    hs[v] += hi;
-    norm_acc(hi, ka, sa[v], ra[v]);
-    if constexpr (TWO) norm_acc(hi, ka - 1, sb[v], rb[v]);
-    if constexpr (TINY) ra[v] = fabsf(x) == 0x1p-75f ? 0.5f : ra[v];
-  }
-  // both binades, with the TINY rule when tiny (the rebuild of k_norm_fix, a binade per chain)
-  __device__ __forceinline__ void add_both(int v, float x, int ka, bool tiny) {
-    const float hi = x * x;
-    norm_acc(hi, ka, sa[v], ra[v]);
-    norm_acc(hi, ka - 1, sb[v], rb[v]);
-    ra[v] = tiny && fabsf(x) == 0x1p-75f ? 0.5f : ra[v];
-  }
-  __device__ __forceinline__ bool tie_a(int v, int) const { return ra[v] == 0.5f; }
-  __device__ __forceinline__ bool tie_b(int v, int) const { return rb[v] == 0.5f; }
-};
-
-// NormAcc of k_norm_seg2d: the ties as per-chain wavefront masks of the lanes that met one (ta, tb;
-// scalar registers), which takes one VALU instruction per element and binade fewer than the largest
-// rounding distance.  (The other record kernels, whose loops are not unrolled, keep NormAcc: their
-// sixteen masks there spill scalar registers.)  Every lane of the wavefront takes part in add.
-struct NormAccM {
-  float sa[8], sb[8], hs[8];
-  uint64_t ta[8], tb[8];
-  __device__ __forceinline__ void clear() {
-#pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      sa[v] = sb[v] = hs[v] = 0.0f;
-      ta[v] = tb[v] = 0;
+  // element x of chain v (TWO: under Ea + 1 too)
+  template <bool TWO>
+  __device__ __forceinline__ void add(int v, float x) {
+    hs[v] = fmaf(x, x, hs[v]);
+    ae[v] = fmaf(x, x, ae[v]);
+    ao[v] = fmaf(x, x, ao[v]);
+    if constexpr (TWO) {
+      be[v] = fmaf(x, x, be[v]);
+      bo[v] = fmaf(x, x, bo[v]);
     }
   }
-  template <bool TWO, bool TINY>
-  __device__ __forceinline__ void add(int v, float x, int ka) {
-    const float hi = x * x;
-    hs[v] += hi;
-    ta[v] |= __ballot(norm_acc_tie(hi, ka, sa[v]));
-    if constexpr (TWO) tb[v] |= __ballot(norm_acc_tie(hi, ka - 1, sb[v]));
-    if constexpr (TINY) ta[v] |= __ballot(fabsf(x) == 0x1p-75f);
-  }
   // An empty asm that reads and writes the sums: in a fully unrolled segment the code generator would
-  // otherwise defer the roundings to the segment's end (their results are read only there) and hold
-  // every square until then.
+  // otherwise interleave chunks and hold their elements longer.
   template <bool TWO>
   __device__ __forceinline__ void pin() {
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      asm volatile("" : "+v"(sa[v]), "+v"(hs[v]), "+s"(ta[v]));
-      if constexpr (TWO) asm volatile("" : "+v"(sb[v]), "+s"(tb[v]));
+      asm volatile("" : "+v"(ae[v]), "+v"(ao[v]), "+v"(hs[v]));
+      if constexpr (TWO) asm volatile("" : "+v"(be[v]), "+v"(bo[v]));
     }
   }
-  __device__ __forceinline__ bool tie_a(int v, int lane) const { return norm_bit(ta[v], lane); }
-  __device__ __forceinline__ bool tie_b(int v, int lane) const { return norm_bit(tb[v], lane); }
+  __device__ __forceinline__ uint32_t val_a(int v, int Ea) const { return norm_lane_value(ae[v], ao[v], Ea); }
+  __device__ __forceinline__ uint32_t val_b(int v, int Ea) const { return norm_lane_value(be[v], bo[v], Ea + 1); }
 };
 
 // The x of the 8 elements at flat index f (a multiple of 8): element v belongs to chain v.  Elements
@@ -520,15 +478,14 @@ __device__ __forceinline__ void norm_chunk_x(const DevTensor& t, int64_t f, int6
   }
 }
 
-// The per-lane, per-chain sums of one segment's increments under the candidate binade (ka = 23 - Ea)
-// and, with TWO, under Ea + 1, with their largest rounding distances and the sums of the squares.
+// Adds chunk steps [h0, h1) of one segment to a lane's sums (TWO: under Ea + 1 too).
 // FULL: the segment holds all kNormSegElems elements.
-template <typename TG, int FORM, bool TWO, bool TINY, bool FULL>
-__device__ __forceinline__ void norm_seg_sums(const DevTensor& t, int64_t f0, int64_t f1, int ka, int lane,
+template <typename TG, int FORM, bool TWO, bool FULL>
+__device__ __forceinline__ void norm_seg_sums(const DevTensor& t, int64_t f0, int64_t f1, int lane,
                                               const Hp& hp, NormAcc& a, int h0 = 0, int h1 = kNormChunks) {
   auto account = [&](const float (&x)[8]) {
 #pragma unroll
-    for (int v = 0; v < 8; ++v) a.add<TWO, TINY>(v, x[v], ka);
+    for (int v = 0; v < 8; ++v) a.add<TWO>(v, x[v]);
   };
   if constexpr (FORM == kNormRows) {
 #pragma unroll 1
@@ -583,8 +540,8 @@ __device__ __forceinline__ void norm_write_records(const DevTensor& t, int64_t s
   float hs[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) {
-    acc[v] = norm_lane_value(a.sa[v], a.tie_a(v, lane), Ea);
-    acc[8 + v] = two ? norm_lane_value(a.sb[v], a.tie_b(v, lane), Ea + 1) : 0u;
+    acc[v] = a.val_a(v, Ea);
+    acc[8 + v] = two ? a.val_b(v, Ea) : 0u;
     hs[v] = a.hs[v];
   }
   norm_lane_sums<8>(hs, lane);    // lane 8c: chain c
@@ -641,9 +598,8 @@ constexpr int kNormSegAhead = 8;       // chunks per lane in flight there
 // the chunk kNormSegAhead on are loaded into the registers this one frees.  Scheduling barriers keep
 // the compiler from hoisting the loads further, and NormAcc::pin keeps each chunk's roundings in its
 // step (either would cost registers, not time).
-template <typename TG, int G, bool TWO, bool TINY, bool ROWS>
-__device__ __forceinline__ void norm_seg_lds(const DevTensor& t, const float* cl, uint32_t f0, int ka, int li,
-                                             NormAccM& a) {
+template <typename TG, int G, bool TWO, bool ROWS>
+__device__ __forceinline__ void norm_seg_lds(const DevTensor& t, const float* cl, uint32_t f0, int li, NormAcc& a) {
   using GS = typename TG::storage;
   constexpr int Q = kNormSegElems / (8 * G), D = kNormSegAhead, NW = int(sizeof(GS)) * 2;
   static_assert(Q >= D, "segment chunks");
@@ -703,11 +659,11 @@ __device__ __forceinline__ void norm_seg_lds(const DevTensor& t, const float* cl
       const uint32_t b = C - cc[s];  // the chunk's elements in its first row
 #pragma unroll
       for (int v = 0; v < 8; ++v)
-        a.add<TWO, TINY>(v, ((uint32_t(v) < b ? r[s] : r1[s]) * cv[v]) * TG::elem(gw[s], v), ka);
+        a.add<TWO>(v, ((uint32_t(v) < b ? r[s] : r1[s]) * cv[v]) * TG::elem(gw[s], v));
       a.template pin<TWO>();
     } else {
 #pragma unroll
-      for (int v = 0; v < 8; ++v) a.add<TWO, TINY>(v, (r[s] * cv[v]) * TG::elem(gw[s], v), ka);
+      for (int v = 0; v < 8; ++v) a.add<TWO>(v, (r[s] * cv[v]) * TG::elem(gw[s], v));
       a.template pin<TWO>();
     }
     if (q + D < Q) issue(s);
@@ -720,14 +676,14 @@ __device__ __forceinline__ void norm_seg_lds(const DevTensor& t, const float* cl
 // were formed (uniform over the wavefront).
 template <int G>
 __device__ __forceinline__ void norm_write_records_g(const DevTensor& t, int64_t seg, int Ea, bool two, bool act,
-                                                     int lane, const NormAccM& a) {
+                                                     int lane, const NormAcc& a) {
   const int li = lane & (G - 1);
   uint32_t acc[16];
   float hs[8];
 #pragma unroll
   for (int v = 0; v < 8; ++v) {
-    acc[v] = norm_lane_value(a.sa[v], a.tie_a(v, lane), Ea);
-    acc[8 + v] = two ? norm_lane_value(a.sb[v], a.tie_b(v, lane), Ea + 1) : 0u;
+    acc[v] = a.val_a(v, Ea);
+    acc[8 + v] = two ? a.val_b(v, Ea) : 0u;
     hs[v] = a.hs[v];
   }
   const int64_t nseg = t.nseg;
@@ -773,8 +729,8 @@ __device__ __forceinline__ void norm_write_records_g(const DevTensor& t, int64_t
 }
 
 // The segments of one wavefront in a run of k_norm_seg2d: segments k0 + sub for k0 = wid * SPW,
-// wid * SPW + 4 * SPW, ... below nrun, sub = lane / G.  TWO and TINY hold for all of them.
-template <typename TG, int G, bool TWO, bool TINY, bool ROWS>
+// wid * SPW + 4 * SPW, ... below nrun, sub = lane / G.  TWO holds for all of them.
+template <typename TG, int G, bool TWO, bool ROWS>
 __device__ __forceinline__ void norm_seg2d_wave(const DevTensor& t, const float* cl, int64_t run0, int64_t nrun,
                                                 float e0, float e1, int wid, int lane) {
   constexpr int SPW = kWave / G;
@@ -788,10 +744,10 @@ __device__ __forceinline__ void norm_seg2d_wave(const DevTensor& t, const float*
     int Ea;
     bool two;
     norm_candidates(e0 + (e1 - e0) * (float(k) / float(nrun)), Ea, two);
-    NormAccM a;
-    a.clear();
+    NormAcc a;
+    a.init(Ea);
     wait_vm_all();  // the previous records' stores: the chunk loads' waits then count only loads
-    norm_seg_lds<TG, G, TWO, TINY, ROWS>(t, cl, uint32_t(seg * kNormSegElems), 23 - Ea, li, a);
+    norm_seg_lds<TG, G, TWO, ROWS>(t, cl, uint32_t(seg * kNormSegElems), li, a);
     norm_write_records_g<G>(t, seg, Ea, TWO, act, lane, a);
   }
 }
@@ -803,8 +759,7 @@ __device__ __forceinline__ void norm_seg2d_wave(const DevTensor& t, const float*
 // segments: the workgroup stages the matrix's column factors in LDS once, and each wavefront takes
 // kWave / kNormSegLanes consecutive segments at a time, a group of kNormSegLanes lanes per segment.
 // A wavefront forms the sums under Ea + 1 for all its segments of the run when one of them needs them
-// (a record with both sums is never wrong), and the subnormal rule when one of them is in that binade;
-// the choice is made once per run, so that no code is shared between the forms' segment loops (the
+// (a record with both sums is never wrong); the choice is made once per run, so that no code is shared between the forms' segment loops (the
 // compiler would hoist a shared start, and the registers it holds, above the branch).
 template <typename TG, int FORM>
 __global__ __launch_bounds__(kThreads) void k_norm_seg2d(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
@@ -837,18 +792,16 @@ __global__ __launch_bounds__(kThreads) void k_norm_seg2d(const DevTensor* __rest
     // the estimate at both ends of the run, linear in between (a chain holds about 1/8 of it)
     const float e0 = uniform_f32(norm_est_at(t, run0 * kNormSegElems)) * 0.125f;
     const float e1 = uniform_f32(norm_est_at(t, min((run0 + nrun) * kNormSegElems, main))) * 0.125f;
-    bool any_two = false, any_tiny = false;
+    bool any_two = false;
     for (int64_t k0 = int64_t(wid) * SPW; k0 < nrun; k0 += (kThreads / kWave) * SPW) {
       const int64_t k = min(k0 + lane / G, nrun - 1);
       int Ea;
       bool two;
       norm_candidates(e0 + (e1 - e0) * (float(k) / float(nrun)), Ea, two);
       any_two |= two;
-      any_tiny |= Ea == -126;
     }
-    if (__any(any_tiny)) norm_seg2d_wave<TG, G, true, true, ROWS>(t, cl, run0, nrun, e0, e1, wid, lane);
-    else if (__any(any_two)) norm_seg2d_wave<TG, G, true, false, ROWS>(t, cl, run0, nrun, e0, e1, wid, lane);
-    else norm_seg2d_wave<TG, G, false, false, ROWS>(t, cl, run0, nrun, e0, e1, wid, lane);
+    if (__any(any_two)) norm_seg2d_wave<TG, G, true, ROWS>(t, cl, run0, nrun, e0, e1, wid, lane);
+    else norm_seg2d_wave<TG, G, false, ROWS>(t, cl, run0, nrun, e0, e1, wid, lane);
   }
 }
 
@@ -877,18 +830,15 @@ __global__ __launch_bounds__(kThreads, 4) void k_norm_seg(const DevTensor* __res
     int Ea;
     bool two;
     norm_candidates(uniform_f32(norm_est_at(t, f0)) * 0.125f, Ea, two);
-    const int ka = 23 - Ea;
     NormAcc a;
-    a.clear();
+    a.init(Ea);
     const bool full = f1 - f0 == kNormSegElems;
-    if (Ea == -126) {
-      norm_seg_sums<TG, FORM, true, true, false>(t, f0, f1, ka, lane, hp, a, h0, h1);
-    } else if (two) {
-      if (full) norm_seg_sums<TG, FORM, true, false, true>(t, f0, f1, ka, lane, hp, a, h0, h1);
-      else norm_seg_sums<TG, FORM, true, false, false>(t, f0, f1, ka, lane, hp, a, h0, h1);
+    if (two) {
+      if (full) norm_seg_sums<TG, FORM, true, true>(t, f0, f1, lane, hp, a, h0, h1);
+      else norm_seg_sums<TG, FORM, true, false>(t, f0, f1, lane, hp, a, h0, h1);
     } else {
-      if (full) norm_seg_sums<TG, FORM, false, false, true>(t, f0, f1, ka, lane, hp, a, h0, h1);
-      else norm_seg_sums<TG, FORM, false, false, false>(t, f0, f1, ka, lane, hp, a, h0, h1);
+      if (full) norm_seg_sums<TG, FORM, false, true>(t, f0, f1, lane, hp, a, h0, h1);
+      else norm_seg_sums<TG, FORM, false, false>(t, f0, f1, lane, hp, a, h0, h1);
     }
     norm_write_records(t, seg, Ea, two, lane, wid, a, xacc, xhs);
   }
@@ -1039,8 +989,8 @@ __device__ __forceinline__ void norm_write_records_pc(const DevTensor& t, int64_
   uint32_t acc[16];
 #pragma unroll
   for (int v = 0; v < 8; ++v) {
-    acc[v] = norm_lane_value(a.sa[v], a.tie_a(v, lane), Ea[v]);
-    acc[8 + v] = norm_lane_value(a.sb[v], a.tie_b(v, lane), Ea[v] + 1);
+    acc[v] = a.val_a(v, Ea[v]);
+    acc[8 + v] = a.val_b(v, Ea[v]);
   }
   norm_lane_sums<16>(acc, lane);  // lane 4c: chain c under Ea[c]; lane 32 + 4c: under Ea[c] + 1
   const int c = (lane >> 2) & 7;
@@ -1126,15 +1076,14 @@ __global__ __launch_bounds__(kThreads) void k_norm_fix(const DevTensor* __restri
     for (int k = wid; k < n; k += kThreads / kWave) {  // uniform over the wavefront
       const uint32_t e = list[k];
       const int64_t sf = base + (e >> 8);
-      int Ea[8], ka[8];
+      int Ea[8];
+      NormAcc a;
 #pragma unroll
       for (int c = 0; c < 8; ++c) {
         bool two;
         norm_candidates(est_l[c][e >> 8], Ea[c], two);
-        ka[c] = 23 - Ea[c];
+        a.init(c, Ea[c]);
       }
-      NormAcc a;
-      a.clear();
       const int64_t f0 = sf * kNormSegElems, f1 = min(f0 + kNormSegElems, main);
       if (kLds && sf < t.nseg0) {  // uniform over the wavefront
 #pragma unroll 1
@@ -1146,7 +1095,7 @@ __global__ __launch_bounds__(kThreads) void k_norm_fix(const DevTensor* __restri
 #pragma unroll
           for (int q = 0; q < kNormGroup; ++q)
 #pragma unroll
-            for (int v = 0; v < 8; ++v) a.add_both(v, x[q][v], ka[v], Ea[v] == -126);
+            for (int v = 0; v < 8; ++v) a.add<true>(v, x[q][v]);
         }
       } else {
 #pragma unroll 1
@@ -1157,7 +1106,7 @@ __global__ __launch_bounds__(kThreads) void k_norm_fix(const DevTensor* __restri
 #pragma unroll
           for (int q = 0; q < kNormGroup; ++q)
 #pragma unroll
-            for (int v = 0; v < 8; ++v) a.add_both(v, x[q][v], ka[v], Ea[v] == -126);
+            for (int v = 0; v < 8; ++v) a.add<true>(v, x[q][v]);
         }
       }
       norm_write_records_pc(t, sf, Ea, e & 255u, lane, a);
