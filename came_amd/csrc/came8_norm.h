@@ -1144,10 +1144,47 @@ __device__ __forceinline__ uint32_t norm_wave_prev(uint32_t incl) { return norm_
 __device__ __forceinline__ uint32_t norm_lane(uint32_t v, int src) { return uint32_t(__builtin_amdgcn_readlane(int(v), src)); }
 __device__ __forceinline__ float norm_lane(float v, int src) { return __uint_as_float(norm_lane(__float_as_uint(v), src)); }
 
+// The x of the 8 elements of a chain at flat indices e0, e0 + 8, ..., e0 + 56 (the first n of them, n <= 8, lie in
+// the segment; the others are 0).  A matrix's rows and columns follow from the first element's by one wrap each
+// (rows of at least 8 elements); other tensors divide for every element.
+template <typename TG>
+__device__ __forceinline__ void norm_x_chain8(const DevTensor& t, int64_t e0, int n, const Hp& hp, float (&x)[8]) {
+  if (t.factored && t.P == 1 && t.idx32 && t.C >= 8) {  // uniform
+    using GS = typename TG::storage;
+    const CAME8_GLOBAL GS* __restrict__ g = gbl(static_cast<const GS*>(t.g));
+    const CAME8_GLOBAL float* __restrict__ rf = gbl(t.rfac);
+    const CAME8_GLOBAL float* __restrict__ cf = gbl(t.cfac);
+    const uint32_t C = uint32_t(t.C), f = uint32_t(e0);
+    uint32_t row = udiv_magic(f, t.mC, t.sC), col = f - row * C;
+    const uint32_t row0 = row, col0 = col;
+    float gv[8], a[8], b[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {  // an element past the segment reads the first one
+      const bool in = j < n;
+      gv[j] = TG::load(g[in ? f + 8u * uint32_t(j) : f]);
+      a[j] = rf[in ? row : row0];
+      b[j] = cf[in ? col : col0];
+      col += 8u;
+      const bool wrap = col >= C;
+      col -= wrap ? C : 0u;
+      row += wrap ? 1u : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = j < n ? (a[j] * b[j]) * gv[j] : 0.0f;
+    return;
+  }
+  int64_t e[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) e[j] = e0 + (j < n ? 8 * j : 0);
+  norm_x_any8<TG>(t, e, hp, x);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = j < n ? x[j] : 0.0f;
+}
+
 // Replays chain c over segment seg from s, equal to the reference's serial fmaf loop bit for bit (one
 // wavefront).  Lane l holds the chain's elements 8l .. 8l + 7 of the segment.  A round takes every
 // remaining element's increment under s's binade, a saturating prefix sum of them in element order,
-// and the first element that is special or whose prefix takes the chain out of the binade; the
+// and the first element that is a tie or whose prefix takes the chain out of the binade; the
 // elements before it are one integer add, that element is one fmaf, and the next round starts after
 // it.  A finite chain only grows, so the rounds are the segment's binade crossings and special
 // elements, plus one.  An infinite chain changes only at a NaN element; a NaN chain not at all.
@@ -1157,19 +1194,10 @@ __device__ float norm_replay(const DevTensor& t, int c, int64_t seg, float s, co
   const int64_t main = t.N - (t.N & 7);
   const int64_t f0 = seg * kNormSegElems;
   const int cnt = int(min(int64_t(kNormChainSeg), (main - f0) / 8));  // at least 1
-  float x[8], h[8];
-  {
-    // an element past the segment's end reads the segment's first element of the chain and counts
-    // for nothing
-    int64_t e[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) e[j] = f0 + 8 * int64_t(lane * 8 + j < cnt ? lane * 8 + j : 0) + c;
-    norm_x_any8<TG>(t, e, hp, x);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = lane * 8 + j < cnt ? x[j] : 0.0f;
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) h[j] = x[j] * x[j];
+  // this lane's elements; a lane wholly past the segment's end reads the segment's first ones and counts for nothing
+  const int mine = min(max(cnt - lane * 8, 0), 8);
+  float x[8];
+  norm_x_chain8<TG>(t, f0 + 64 * int64_t(mine > 0 ? lane : 0) + c, mine, hp, x);
   if (s == 0.0f) {
     // A chain's first segment crosses a binade every few elements, and its early increments keep many
     // fractional bits, so ties are common too: instead of a round per crossing or tie, its elements are
@@ -1207,28 +1235,23 @@ __device__ float norm_replay(const DevTensor& t, int c, int64_t seg, float s, co
     const int E = norm_binade(s);
     const uint32_t m = norm_mant(s, E);
     const uint32_t room = kNormFull - m;  // an increment prefix that reaches this leaves the binade
-    const int kk = 23 - E;
-    uint32_t incl[8], spm = 0, run = 0;
+    // this lane's increments as prefixes, from the pair of sums of the records (NormAcc); the first tie or
+    // departure from the binade within the lane is an event, after which its prefixes mean nothing
+    const uint32_t bits = uint32_t(E + 127) << 23;
+    float even = __uint_as_float(bits), odd = __uint_as_float(bits + 1u);
+    uint32_t incl[8], evm = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const int k = lane * 8 + j;
-      const bool live = k >= pos && k < cnt;
-      const float dh = ldexpf(h[j], kk);
-      const float nf = rintf(dh);
-      const bool special = fabsf(dh - nf) == 0.5f || (E == -126 && (nf != 0.0f || fabsf(x[j]) == 0x1p-75f));
-      const uint32_t n = nf < 0x1p25f ? uint32_t(nf) : kNormSat;  // NaN and inf squares saturate
-      run = sat_add(run, live ? n : 0u);
-      incl[j] = run;
-      spm |= (live && special) ? (1u << j) : 0u;
+      const float xj = lane * 8 + j >= pos ? x[j] : 0.0f;  // (elements past the segment's end are 0)
+      even = fmaf(xj, xj, even);
+      odd = fmaf(xj, xj, odd);
+      incl[j] = __float_as_uint(even) - bits;
+      evm |= (incl[j] >= (1u << 23) || __float_as_uint(odd) - bits != incl[j] + 1u) ? (1u << j) : 0u;
     }
-    const uint32_t winc = norm_wave_scan(run);  // inclusive scan of the lanes' runs
+    const uint32_t winc = norm_wave_scan(min(incl[7], kNormSat));  // inclusive scan of the lanes' runs
     const uint32_t excl = norm_wave_prev(winc);
-    uint32_t evm = spm;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int k = lane * 8 + j;
-      evm |= (k >= pos && k < cnt && sat_add(excl, incl[j]) >= room) ? (1u << j) : 0u;
-    }
+    for (int j = 0; j < 8; ++j) evm |= excl + min(incl[j], kNormSat) >= room ? (1u << j) : 0u;
     const uint64_t bal = __ballot(evm != 0);
     if (bal == 0) {
       s = norm_value(m + norm_lane(winc, kWave - 1), E);  // below room
