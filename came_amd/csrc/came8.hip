@@ -111,6 +111,8 @@ struct Plan {
   std::map<int, WorkList> tiny1;         // P1 of tensors of tiny matrices (per ngrp matrices), by grad type
   std::map<int, WorkList> tiny2;         // P2 of tensors of tiny matrices, by grad type
   WorkList tinyq;                        // their states' codes (per four state blocks)
+  // small tensors, a workgroup each for the whole step, by types: up to kSmallElems elements, and larger ones
+  std::map<TypeKey, WorkList> smallS, smallL;
   std::map<TypeKey, WorkList> upd;       // P3, tile form (fast block sizes)
   std::map<TypeKey, WorkList> updb;      // P3, band form
   std::map<TypeKey, WorkList> vecB;      // 1-D pass B (fast block sizes)
@@ -157,6 +159,7 @@ bool fast_block(int B) { return B >= 8 && B <= kTile && (B & (B - 1)) == 0; }
 // rows per work item of the band form of P3 (at most).  Measured on C4 / C2 pass 3: 4 rows 10.69 / 0.948 ms,
 // 8 rows 10.37 / 0.923, 16 rows 10.48 / 0.948, 32 rows 10.55 (C4), 64 rows 10.90 (C4)
 constexpr int kP3BandRows = 8;
+constexpr int64_t kOneRoundSmall = 256;  // small tensors of one launch of the larger size at most: one a CU
 constexpr int64_t kP3MinItems = 1024;  // band-form P3 work items wanted per launch (4 per CU)
 constexpr int64_t kP3BandMinCols = 1024;  // narrower rows leave too many of a workgroup's lanes idle
 // The clip-norm walk takes 12-17 ns per segment of a tensor's chain and runs serially along it; below
@@ -233,6 +236,22 @@ void magic_div(int64_t d, uint64_t& m, uint32_t& s) {
 // takes the thread-per-matrix passes.
 bool tiny_matrix(const came8_tensor& t, bool s2d) {
   return t.factored && !s2d && t.rows >= 1 && t.cols >= 1 && t.rows * t.cols <= kTinyElems;
+}
+
+// A tensor whose whole step one workgroup can do (k_small_step).
+bool small_tensor(const came8_tensor& t) {
+  if (t.state_kind == CAME8_STATE_8BIT2D || t.rows < 1 || t.cols < 1 || t.prefix != 1) return false;
+  if (t.rows > kLargeElems || t.cols > kLargeElems || t.rows * t.cols > kLargeElems) return false;
+  return !t.factored || t.rows + t.cols <= kSmallStates;
+}
+
+// The tensors take k_small_step when all of them can: beside larger tensors they ride along in launches that are made
+// anyway, at less than the 20 us that kernel takes for a vector of 2048 (292 tensors of a 24-layer model: 1965 us, 1986
+// with its 194 vectors in a launch of their own).
+bool all_small(const came8_tensor* ts, int32_t n) {
+  for (int32_t i = 0; i < n; ++i)
+    if (!small_tensor(ts[i])) return false;
+  return true;
 }
 
 // Matrices per work item of those passes, and per unit of the clip-norm estimates (at most kNormMaxUnits of them)
@@ -359,7 +378,7 @@ std::vector<int> band_shrinks(const came8_tensor* ts, int32_t n, int32_t B) {
               elems.push_back(double(std::min(rb, t.rows - bnd * rb)) * double(t.cols));
           partial += 3.0 * double(t.prefix * nb) * double(t.cols);
         }
-        if (rb_sum == prev_rb_sum) break;  // every band is at its least height already
+        if (rb_sum == prev_rb_sum) continue;  // the same bands again (of at least 8 rows, or of whole matrices)
         prev_rb_sum = rb_sum;
         // one pass: the busiest workgroup's elements, at 1/slots of the GPU's rate
         auto pass_time = [&](int64_t slots) {
@@ -388,10 +407,11 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
   if (n > 0 && ts == nullptr) return fail(CAME8_EINVAL, "came8: tensors is NULL");
   if (B <= 0) return fail(CAME8_EINVAL, "came8: block_size must be > 0, got " + std::to_string(B));
   plan.dev.assign(n, DevTensor{});
+  const bool small = all_small(ts, n);
   // --- scratch layout (after the plan blob; offsets relative to the scratch start) ---
   std::vector<size_t> scr_off(n, 0);
   size_t scr = 0;
-  const std::vector<int> shrink = (B > 0 && n > 0) ? band_shrinks(ts, n, B) : std::vector<int>(std::max(n, 0), 0);
+  const std::vector<int> shrink = (B > 0 && n > 0 && !small) ? band_shrinks(ts, n, B) : std::vector<int>(std::max(n, 0), 0);
   for (int i = 0; i < n; ++i) {
     const came8_tensor& t = ts[i];
     const std::string who = "came8: tensor " + std::to_string(i) + ": ";
@@ -483,7 +503,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     d.p3_rb = 0;
     d.p3_nseg = 0;
     d.p3_nbands = 0;
-    if (t.factored && !s2d && fast_block(B) && d.rowal && d.vec_ok && d.C >= kP3BandMinCols) {
+    if (t.factored && !s2d && !small && fast_block(B) && d.rowal && d.vec_ok && d.C >= kP3BandMinCols) {
       const int64_t bpr = d.C / B, bmax = kTile / B;  // blocks per row, per segment
       d.p3_nseg = int32_t(ceil_div(bpr, bmax));
       d.p3_rb = kP3BandRows;
@@ -491,7 +511,13 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     }
     magic_div(d.C, d.mC, d.sC);
     magic_div(d.R, d.mR, d.sR);
-    if (t.factored) {
+    if (small) {  // one workgroup's step keeps everything but the clip divisor on chip
+      d.rb = d.R;
+      d.nbands = 1;
+      d.nbr = t.factored ? std::max<int64_t>(1, ceil_div(d.R, B)) : d.nbm;
+      d.nbc = t.factored ? std::max<int64_t>(1, ceil_div(d.C, B)) : 0;
+      o.clip = take(8);
+    } else if (t.factored) {
       d.rb = tiny_matrix(t, s2d) ? d.R : band_rows(d.R, d.C, shrink[i]);
       d.nbands = ceil_div(d.R, d.rb);
       d.nbr = d.pm ? d.P * d.pmb_r : std::max<int64_t>(1, ceil_div(d.P * d.R, B));
@@ -534,7 +560,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     d.nrun = kNormRunSegs;
     d.nunit = 0;
     d.ngrp = 1;
-    if (!s2d) {
+    if (!s2d && !small) {
       d.nseg = ceil_div(d.N - (d.N & 7), kNormSegElems);
       const bool lds = t.factored && d.idx32 && reinterpret_cast<uintptr_t>(t.grad) % 16 == 0 && d.P == 1 &&
                        !tiny_matrix(t, false) && d.C >= 8 * kNormSegLanes && d.C + (d.c8 ? 0 : 8) <= kNormLdsCols;
@@ -557,7 +583,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     scr_off[i] = scr;
     // store offsets temporarily as integers in the pointer fields (rebased below)
     auto at = [&](size_t x) { return reinterpret_cast<float*>(scr + x); };
-    if (t.factored) {
+    if (t.factored && !small) {
       d.Rn = at(o.Rn); d.rfac = at(o.rfac); d.RRn = at(o.RRn); d.rrfac = at(o.rrfac);
       d.Cn = at(o.Cn); d.cfac = at(o.cfac); d.CRn = at(o.CRn); d.crfac = at(o.crfac);
       d.partU = at(o.pU); d.partW = at(o.pW);
@@ -573,7 +599,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     }
     d.clip_part = reinterpret_cast<double*>(scr + o.clipp);
     d.clip = at(o.clip);
-    if (!s2d) {
+    if (!s2d && !small) {
       d.nest = at(o.nest);
       d.nrec = reinterpret_cast<uint32_t*>(scr + o.nrec);
       d.nsum = at(o.nsum);
@@ -635,6 +661,10 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     const came8_tensor& t = ts[i];
     const DevTensor& d = plan.dev[i];
     const TypeKey tk{t.param_dtype, t.grad_dtype, d.fp32st};
+    if (small) {
+      add_item((d.N <= kSmallElems ? plan.smallS : plan.smallL)[TypeKey{t.param_dtype, t.grad_dtype, 0}], i, 1);
+      continue;
+    }
     if (d.mode2d) {
       const BandShapeSel sel = band_variant(t, d.C, B, 1);
       add_item(plan.band2dw[BandKey{t.grad_dtype, sel.V, sel.K, sel.TPB, 0, sel.ua}], i, d.nbands);
@@ -704,6 +734,14 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     add_item((longc[i] ? plan.nfinalL : plan.nfinal)[t.grad_dtype], i, 1);
   }
 
+  // a few tensors of both sizes: one launch of the larger size, a workgroup a CU
+  for (auto& kv : plan.smallL) {
+    auto it = plan.smallS.find(kv.first);
+    if (it == plan.smallS.end() || it->second.total() + kv.second.total() > kOneRoundSmall) continue;
+    for (int32_t ti : it->second.tids) add_item(kv.second, ti, 1);
+    plan.smallS.erase(it);
+  }
+
   // --- blob: DevTensor[n] then every work list (tids, wstart) ---
   size_t off = align_up(sizeof(DevTensor) * size_t(n), 16);
   auto place = [&](WorkList& wl) {
@@ -725,6 +763,8 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
   for (auto& kv : plan.param2d) place(kv.second);
   place(plan.res2d);
   place(plan.tinyq);
+  for (auto& kv : plan.smallS) place(kv.second);
+  for (auto& kv : plan.smallL) place(kv.second);
   for (auto& kv : plan.upd) place(kv.second);
   for (auto& kv : plan.updb) place(kv.second);
   for (auto& kv : plan.vecB) place(kv.second);
@@ -757,6 +797,10 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     };
     for (int i = 0; i < n; ++i) {
       DevTensor& d = plan.dev[i];
+      if (small) {
+        rebase(d.clip);
+        continue;
+      }
       if (d.factored) {
         rebase(d.Rn); rebase(d.rfac); rebase(d.RRn); rebase(d.rrfac);
         rebase(d.Cn); rebase(d.cfac); rebase(d.CRn); rebase(d.crfac);
@@ -800,6 +844,8 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     for (auto& kv : plan.param2d) put(kv.second);
     put(plan.res2d);
     put(plan.tinyq);
+    for (auto& kv : plan.smallS) put(kv.second);
+    for (auto& kv : plan.smallL) put(kv.second);
     for (auto& kv : plan.upd) put(kv.second);
     for (auto& kv : plan.updb) put(kv.second);
     for (auto& kv : plan.vecB) put(kv.second);
@@ -919,6 +965,12 @@ BandFn band_fn(int gdt, bool pass2, int V, int K, int TPB, int st, int ua, int m
 }
 
 using GenFn = void (*)(const DevTensor*, const int32_t*, const int64_t*, int, Hp);
+using SmallFn = void (*)(const DevTensor*, const int32_t*, int, int, Hp);
+
+template <typename TP, typename TG>
+constexpr SmallFn k_small_step_S = k_small_step<TP, TG, kSmallThreads>;
+template <typename TP, typename TG>
+constexpr SmallFn k_small_step_L = k_small_step<TP, TG, kLargeThreads>;
 
 template <typename TP, typename TG>
 constexpr GenFn k_fact_pass3_q8 = k_fact_pass3<TP, TG, false>;
@@ -1016,11 +1068,11 @@ int check_launch(const char* what) {
 const char* const kPhaseNames[] = {"pass1", "vec_passA", "row_mean", "factor_blocks", "clip", "norm_est",
                                    "pass2", "row_mean_res", "factor_blocks_res", "pass3", "vec_passB",
                                    "generic_update", "tiles2d", "res_rows2d", "param2d", "norm_bsum",
-                                   "norm_seg", "norm_walk", "norm_final", "norm_fix"};
+                                   "norm_seg", "norm_walk", "norm_final", "norm_fix", "small_step"};
 constexpr int kNumPhases = sizeof(kPhaseNames) / sizeof(kPhaseNames[0]);
 enum Phase { PH_PASS1, PH_VECA, PH_ROWMEAN, PH_FACTOR, PH_CLIP, PH_NORM_EST, PH_PASS2, PH_ROWMEAN_RES,
              PH_FACTOR_RES, PH_PASS3, PH_VECB, PH_GENERIC, PH_TILES2D, PH_RES2D, PH_PARAM2D, PH_NORM_BSUM,
-             PH_NORM_SEG, PH_NORM_WALK, PH_NORM_FINAL, PH_NORM_FIX };
+             PH_NORM_SEG, PH_NORM_WALK, PH_NORM_FINAL, PH_NORM_FIX, PH_SMALL };
 
 struct Pending {
   int phase;
@@ -1252,6 +1304,11 @@ double alg_bytes(const Plan& plan, const WorkList& wl, const came8_tensor* ts, i
       case PH_PARAM2D:  // m, tile scales, p rw (weight decay folded in)
         tot += N * (1.0 + 2.0 * sp) + 4.0 * double(d.tr) * double(d.tc);
         (void)wd;
+        break;
+      case PH_SMALL:  // g, p rw, m rw, and the second-moment (and residual) states rw
+        tot += N * (sg + 2.0 * sp + 2.0 * mb) + (d.fp32st ? 0.0 : 8.0 * nbm);
+        if (d.factored) tot += 4.0 * vb * double(d.R + d.C) + (d.fp32st ? 0.0 : 16.0 * double(d.nbr + d.nbc));
+        else tot += 2.0 * N * vb + (d.fp32st ? 0.0 : 8.0 * nbm);
         break;
       case PH_NORM_SEG: tot += N * sg; break;  // g (the factors come from cache)
       case PH_FACTOR: case PH_FACTOR_RES:  // one row + one column state: codes rw, scales rw
@@ -1513,6 +1570,26 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
   };
   bool split = false;  // the long-chain group runs on the side stream (set by the clip-norm section)
 
+  // ---- small tensors: the whole step ----
+  for (const bool large : {false, true}) {
+    for (auto& kv : large ? plan.smallL : plan.smallS) {
+      const WorkList& wl = kv.second;
+      SmallFn fn;
+      if (large) CAME8_TYPE_SWITCH2(k_small_step_L, kv.first.pdt, kv.first.gdt, fn);
+      else CAME8_TYPE_SWITCH2(k_small_step_S, kv.first.pdt, kv.first.gdt, fn);
+      const int nt = large ? kLargeThreads : kSmallThreads;
+      size_t lds = 0;
+      for (int32_t ti : wl.tids) {
+        const DevTensor& d = plan.dev[ti];
+        lds = std::max(lds, small_lds(nt, d.N, d.factored ? d.R + d.C : 0));
+      }
+      PhaseTimer pt(PH_SMALL, alg_bytes(plan, wl, tensors, PH_SMALL), stream);
+      hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), dim3(nt), lds, stream, dT, tids(wl), int(wl.tids.size()),
+                         int(exact_norm), hp);
+      if ((rc = check_launch("small_step")) != CAME8_OK) return rc;
+    }
+  }
+
   // ---- P1 and 1-D pass A ----
   // the default clip mode's pass 1 keeps no column sums of g^2/R_i (k_fact_pass1n), except for the
   // 8bit2d tensors, whose clip is formed from them
@@ -1644,7 +1721,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     }
     if ((rc = launch_walk(plan.nwalk, plan.nfinal, stream)) != CAME8_OK) return rc;
   }
-  if (exact_norm || any2d) {  // reference order: only the 8bit2d tensors take this divisor
+  if ((exact_norm && (any_fact || !plan.vecA.empty())) || any2d) {  // reference order: only the 8bit2d tensors take this divisor
     PhaseTimer pt(PH_CLIP, 0.0, stream);
     hipLaunchKernelGGL(k_clip<>, dim3(grid_for(n_tensors)), blk, 0, stream, dT, int(n_tensors), int(!exact_norm), hp);
     if ((rc = check_launch("clip")) != CAME8_OK) return rc;

@@ -1203,10 +1203,13 @@ __device__ float norm_replay(const DevTensor& t, int c, int64_t seg, float s, co
     // fractional bits, so ties are common too: instead of a round per crossing or tie, its elements are
     // applied one by one (the reference's own loop), each broadcast from its lane.  Elements past the
     // segment's end are 0, and fmaf(0, 0, s) is s, so the loop needs no branch.
+#pragma unroll 1
+    for (int l = 0; l < kWave; l += 2) {  // (unrolled whole, the loop's code takes longer to fetch than to run)
 #pragma unroll
-    for (int k = 0; k < kNormChainSeg; ++k) {
-      const float xk = norm_lane(x[k & 7], k >> 3);
-      s = fmaf(xk, xk, s);
+      for (int k = 0; k < 16; ++k) {
+        const float xk = norm_lane(x[k & 7], l + (k >> 3));
+        s = fmaf(xk, xk, s);
+      }
     }
     return s;
   }
@@ -1415,6 +1418,352 @@ __global__ __launch_bounds__(kThreads) void k_norm_final(const DevTensor* __rest
   const float c = clip_from_norm(sqrtf(b), t.N, hp);
   t.clip[0] = c;
   t.clip[1] = rcp_for_div(c);
+}
+
+// ---------------------------------------------------------------------------
+// small tensors: the whole step in one workgroup
+// ---------------------------------------------------------------------------
+// A 1-D tensor or a matrix (prefix 1) of at most kLargeElems elements with at most kSmallStates rows and columns takes
+// one workgroup for all of its step: the passes above are a dozen dependent launches of a few microseconds each, which
+// is all the time a small tensor takes (a 96x200 layer, a 16x1280 adapter: 5 to 15 us a launch, 150 us a step).  The
+// update (then u - m, then m) stays in LDS, where the sums over rows and columns and the eight serial chains of the clip
+// norm read it; a matrix's momentum is formed twice, as in the passes, since LDS holds one float an element.  The
+// arithmetic is that of the passes.  What bounds it is latency: the chains (4.6 ns an element of one), a memory round
+// trip per eight elements of a thread and operand, and the sums.  Two sizes: 256 threads for up to kSmallElems elements,
+// several workgroups a CU, and 1024 threads, whose LDS may fill a CU.  A step of 96x200, 96, 10x96 and 10: 161 us in
+// twelve launches, 61 in this one; 192 adapters of 16x640 to 16x2048: 333 us in 17, 95 in this one.
+constexpr int kSmallThreads = 256, kLargeThreads = 1024;
+constexpr int kSmallElems = 2048, kLargeElems = 32768;
+constexpr int64_t kSmallStates = 2560;  // rows + columns: two floats each beside kLargeElems floats of LDS
+// LDS of a workgroup of nt threads for tensors of up to n elements and s states
+constexpr size_t small_lds(int nt, int64_t n, int64_t s) { return size_t(nt) * 8 + size_t(n) * 4 + size_t(s) * 8; }
+
+// Sums over the rows and the columns of val(e)^2 of an R x C matrix, in fp64 and a fixed order; row(r, s) and
+// col(j, s) are each called by one thread.  Four values at a time, so that their loads overlap (past the end: a value
+// that exists, counted as zero).  dsum: NT doubles of LDS.  Every thread calls it; it synchronises before the columns
+// are finished, not after.
+template <typename Val>
+__device__ __forceinline__ double small_sum4(Val val, int e0, int step, int n) {  // n values from e0, step apart
+  double s = 0.0;
+#pragma unroll 1
+  for (int i = 0; i < n; i += 4) {
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = val(e0 + min(i + k, n - 1) * step);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double d = i + k < n ? double(v[k]) : 0.0;
+      s = fma(d, d, s);
+    }
+  }
+  return s;
+}
+template <int NT, typename Val, typename RowFn, typename ColFn>
+__device__ __forceinline__ void small_sums(Val val, int R, int C, double* dsum, RowFn row, ColFn col) {
+  const int tid = threadIdx.x;
+  int lg = 0;  // 2^lg lanes of a row: about four values each
+  while (lg < 6 && (4 << lg) < C) ++lg;
+  const int G = 1 << lg, li = tid & (G - 1);
+  for (int r0 = 0; r0 < R; r0 += NT >> lg) {  // uniform
+    const int r = r0 + (tid >> lg);
+    double s = 0.0;
+    if (r < R && li < C) s = small_sum4(val, r * C + li, G, (C - li + G - 1) >> lg);
+    for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, kWave);
+    if (r < R && li == 0) row(r, s);
+  }
+  if (C >= NT) {
+    for (int j = tid; j < C; j += NT) col(j, small_sum4(val, j, C, R));
+    __syncthreads();
+  } else {
+    const int H = min(kWave, NT / C);  // threads of a column, every H-th row each
+    const int h = tid / C, j = tid - h * C;
+    if (h < H) dsum[tid] = h < R ? small_sum4(val, h * C + j, H * C, (R - h + H - 1) / H) : 0.0;
+    __syncthreads();
+    if (tid < C) {
+      double s = dsum[tid];
+      for (int k = 1; k < H; ++k) s += dsum[k * C + tid];
+      col(tid, s);
+    }
+  }
+}
+
+// Codes and scales of n values in LDS, a wavefront per block of B (any size; a short block is zero padded).  A lane
+// holds its first four values of a block (all of them up to B = 256).
+template <bool SIGNED, int NW>
+__device__ __forceinline__ void small_quant(const float* x, int n, int B, void* q, float* a) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int nb = (n + B - 1) / B;
+  CAME8_GLOBAL uint8_t* qb = gbl(static_cast<uint8_t*>(q));
+#pragma unroll 1
+  for (int blk = wid; blk < nb; blk += NW) {
+    const int i0 = blk * B, i1 = min(i0 + B, n);
+    float v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = x[min(i0 + lane + k * kWave, i1 - 1)];  // past the end: the last one again
+    float mx = nan_max(nan_max(quant_val<SIGNED>(v[0]), quant_val<SIGNED>(v[1])),
+                       nan_max(quant_val<SIGNED>(v[2]), quant_val<SIGNED>(v[3])));
+    if (!SIGNED && i1 - i0 < B) mx = nan_max(mx, 0.0f);
+    for (int i = i0 + lane + 4 * kWave; i < i1; i += kWave) mx = nan_max(mx, quant_val<SIGNED>(x[i]));
+    const float raw = group_max<64>(mx), am = fix_absmax(raw), rcp = rcp_for_div(am);
+    const bool fast = rcp == rcp && raw == raw;
+    uint32_t c[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) c[k] = quant_code<SIGNED>(v[k], am, rcp, fast);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (i0 + lane + k * kWave < i1) qb[i0 + lane + k * kWave] = uint8_t(c[k]);
+    for (int i = i0 + lane + 4 * kWave; i < i1; i += kWave) qb[i] = uint8_t(quant_code<SIGNED>(x[i], am, rcp, fast));
+    if (lane == 0) a[blk] = am;
+  }
+}
+
+// sum over the workgroup of one double a thread, in a fixed order (every thread gets it; synchronises)
+template <int NT>
+__device__ __forceinline__ double small_total(double v, double* dsum) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  v = wave_sum(v);
+  __syncthreads();  // dsum's readers are done
+  if (lane == 0) dsum[wid] = v;
+  __syncthreads();
+  double s = dsum[0];
+#pragma unroll
+  for (int k = 1; k < NT / kWave; ++k) s += dsum[k];
+  return s;
+}
+
+// This thread's elements e = tid, tid + NT, ... of an R x C matrix (or a row of C), U at a time: load(e, k) of all U,
+// then calc(row, col, k) of all, then store(e, k) of those that exist (the others are the last element again).
+template <int NT, int U, typename Load, typename Calc, typename Store>
+__device__ __forceinline__ void small_each(int N, int R, int C, Load load, Calc calc, Store store) {
+  const int tid = threadIdx.x;
+  int row = tid / C, col = tid - row * C;
+  const int dq = NT / C, dr = NT - dq * C;  // the next element's row and column follow from this one's
+#pragma unroll 1
+  for (int e0 = tid; e0 < N; e0 += U * NT) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) load(uint32_t(min(e0 + k * NT, N - 1)), k);
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      calc(min(row, R - 1), col, k);
+      row += dq;
+      col += dr;
+      const bool wrap = col >= C;
+      col -= wrap ? C : 0;
+      row += wrap ? 1 : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (e0 + k * NT < N) store(uint32_t(e0 + k * NT), k);
+  }
+}
+
+template <typename TP, typename TG, int NT>
+__global__ __launch_bounds__(NT) void k_small_step(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
+                                                   int ntens, int exact_norm, Hp hp) {
+  using GS = typename TG::storage;
+  using PS = typename TP::storage;
+  extern __shared__ double small_mem[];
+  __shared__ float clip_s;
+  constexpr int NW = NT / kWave;
+  constexpr int U = 8;  // elements a thread loads together
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int item = blockIdx.x; item < ntens; item += gridDim.x) {
+    const DevTensor& t = T[tids[item]];
+    const bool fact = t.factored != 0, f32 = t.fp32st != 0;
+    const int N = int(t.N), R = int(t.R), C = int(t.C);
+    double* dsum = small_mem;
+    float* x = reinterpret_cast<float*>(small_mem + NT);  // N
+    float* fac = x + N;                                   // row factors r_i [R], column factors c_j [C]
+    float* stv = fac + (fact ? R + C : 0);                // the new states, alike; then rr_i, cr_j
+    const CAME8_GLOBAL GS* __restrict__ g = gbl(static_cast<const GS*>(t.g));
+    const CAME8_GLOBAL float* m32 = gbl(static_cast<const float*>(st_m(t)));
+    const CAME8_GLOBAL int8_t* mq = gbl(static_cast<const int8_t*>(t.mq));
+    const CAME8_GLOBAL float* ma = gbl(static_cast<const float*>(t.ma));
+    const CAME8_GLOBAL float* v32 = gbl(static_cast<const float*>(st_sq_row(t)));
+    const CAME8_GLOBAL uint8_t* vq = gbl(static_cast<const uint8_t*>(t.rq));
+    const CAME8_GLOBAL float* va = gbl(static_cast<const float*>(t.ra));
+    // e / B for e < 2^15: the quotient of e + 1/2 is at least 1 / (2B) from a whole number, its error below 2^-8 / B
+    const float invB = 1.0f / float(hp.B);
+    auto blk = [&](uint32_t e) __attribute__((always_inline)) { return uint32_t((float(e) + 0.5f) * invB); };
+    // the old momentum of element e of the 8-bit states (no branch, which would make several elements' loads wait for
+    // each other: an infinite or NaN scale / 127 is itself)
+    auto m_q8 = [&](uint32_t e) __attribute__((always_inline)) {
+      const float a = ma[blk(e)];
+      return float(mq[e]) * (fabsf(a) <= 0x1.fffffep127f ? div_fast(a, kSignedQ, kRcpSignedQ) : a);
+    };
+    // the row and column states (RES: of the residual) from the sums of the squares in x: the new states into stv and
+    // to memory (codes and scales, or fp32 states), factors into fac (RES: over the states in stv).  Ends synchronised.
+    auto states = [&](auto RES) __attribute__((always_inline)) {
+      constexpr bool kRes = decltype(RES)::value;
+      const float beta = kRes ? hp.b3 : hp.b2, alpha = kRes ? hp.a3 : hp.a2;
+      const double eps = double(kRes ? hp.eps1 : hp.eps0);
+      const float fC = float(C), fR = float(R), invC = 1.0f / fC;
+      float* rst = kRes ? t.ra : st_sq_row(t);  // fp32 states
+      float* cst = kRes ? t.ca : st_sq_col(t);
+      uint8_t* rq = t.rq + (kRes ? R : 0);
+      uint8_t* cq = t.cq + (kRes ? C : 0);
+      float* ra = t.ra + (kRes ? t.nbr : 0);
+      float* ca = t.ca + (kRes ? t.nbc : 0);
+      double rs = 0.0;
+      small_sums<NT>([&](int e) { return x[e]; }, R, C, dsum, [&](int r, double s) {
+        const float old = f32 ? rst[r] : deq_u8(rq[r], ra[blk_of(r, hp)]);
+        const float tot = float(s + double(C) * eps);
+        const float v = fmaf(kRes ? tot / fC : tot * invC, alpha, old * beta);
+        stv[r] = v;
+        rs += v;
+      }, [&](int j, double s) {
+        const float old = f32 ? cst[j] : deq_u8(cq[j], ca[blk_of(j, hp)]);
+        stv[R + j] = clamp_min_tiny(fmaf(float(s + double(R) * eps) / fR, alpha, old * beta));
+      });
+      const float mean = row_mean_of_sum(t, small_total<NT>(rs, dsum));  // synchronises: stv is whole
+      if constexpr (!kRes)
+        for (int r = tid; r < R + C; r += NT) fac[r] = rsqrt_ref(r < R ? stv[r] / mean : stv[r]);
+      if (f32) {
+        for (int r = tid; r < R; r += NT) rst[r] = stv[r];
+        for (int j = tid; j < C; j += NT) cst[j] = stv[R + j];
+      } else {  // (every old code was read before the barriers above)
+        small_quant<false, NW>(stv, R, hp.B, rq, ra);
+        small_quant<false, NW>(stv + R, C, hp.B, cq, ca);
+      }
+      __syncthreads();
+      if constexpr (kRes) {
+        for (int r = tid; r < R + C; r += NT) stv[r] = rsqrt_ref(r < R ? stv[r] / mean : stv[r]);
+        __syncthreads();
+      }
+    };
+    // ---- the update, into x ----
+    float gv[U], vo[U];
+    auto load_v = [&](uint32_t e, int k) __attribute__((always_inline)) {  // a 1-D tensor's gradient and old second moment
+      gv[k] = TG::load(g[e]);
+      vo[k] = f32 ? v32[e] : deq_u8(vq[e], va[blk(e)]);
+    };
+    if (fact) {
+      small_each<NT, U>(N, R, C, [&](uint32_t e, int k) { gv[k] = TG::load(g[e]); }, [](int, int, int) {},
+                        [&](uint32_t e, int k) { x[e] = gv[k]; });
+      __syncthreads();
+      states(std::false_type{});
+      small_each<NT, U>(N, R, C, [&](uint32_t e, int k) { gv[k] = x[e]; },
+                        [&](int row, int col, int k) { gv[k] = (fac[row] * fac[R + col]) * gv[k]; },
+                        [&](uint32_t e, int k) { x[e] = gv[k]; });
+    } else {
+      small_each<NT, U>(N, 1, N, load_v, [&](int, int, int k) { gv[k] = rsqrt_ref(vec_v_from(gv[k], vo[k], hp)) * gv[k]; },
+                        [&](uint32_t e, int k) { x[e] = gv[k]; });
+    }
+    __syncthreads();
+    // ---- the clip divisor ----
+    float norm = 0.0f;
+    if (exact_norm) {
+      double s = 0.0;
+      for (int e = tid; e < N; e += NT) s = fma(double(x[e]), double(x[e]), s);
+      norm = float(sqrt(small_total<NT>(s, dsum)));
+    } else if (tid < kWave) {  // lane c < 8: chain c; then the chains and the tail in the reference's order (k_norm_final)
+      const int n8 = N >> 3;
+      const float* xc = x + (lane & 7);
+      float acc = 0.0f;
+      // 16 elements load while the 16 before them are added
+      auto load16 = [&](float (&y)[16], int i) __attribute__((always_inline)) {
+        const int j = i + 16 <= n8 ? i : 0;  // past the end: unused
+#pragma unroll
+        for (int k = 0; k < 16; ++k) y[k] = xc[(j + k) * 8];
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto add16 = [&](const float (&y)[16]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 16; ++k) acc = fmaf(y[k], y[k], acc);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      int i = 0;
+      if (n8 >= 16) {
+        float y[16], z[16];
+        load16(y, 0);
+#pragma unroll 1
+        for (; i + 32 <= n8; i += 32) {
+          load16(z, i + 16);
+          add16(y);
+          load16(y, i + 32);
+          add16(z);
+        }
+        if (i + 16 <= n8) {
+          add16(y);
+          i += 16;
+        }
+      }
+      for (; i < n8; ++i) acc = fmaf(xc[i * 8], xc[i * 8], acc);
+      float b = norm_lane(acc, 0);
+#pragma unroll
+      for (int k = 1; k < 8; ++k) b = b + norm_lane(acc, k);
+      int d = n8 * 8;
+      if (N - d >= 4) {
+        for (const int e = d + 4; d < e; ++d) {
+          const float sq = x[d] * x[d];
+          b = b + sq;
+        }
+      }
+      for (; d < N; ++d) b = fmaf(x[d], x[d], b);
+      norm = sqrtf(b);
+    }
+    if (tid == 0) {
+      const float c = clip_from_norm(norm, t.N, hp);
+      clip_s = c;
+      t.clip[0] = c;
+      t.clip[1] = rcp_for_div(c);
+    }
+    __syncthreads();
+    const float clip = clip_s;
+    // ---- the momentum: a vector's into x; of a matrix d = u - m for the residual's sums, and again for the write ----
+    const bool h16 = !fact && !f32 && (hp.fp16u || t.fp16u);
+    auto m_new = [&](float w, float mo) { return fmaf(w, hp.a1, mo * hp.b1); };
+    float mo[U];
+    small_each<NT, U>(N, 1, N, [&](uint32_t e, int k) {
+      mo[k] = f32 ? m32[e] : m_q8(e);
+      gv[k] = x[e];
+    }, [&](int, int, int k) {
+      const float w = (h16 ? round_f16(gv[k]) : gv[k]) / clip;
+      const float m = m_new(w, mo[k]);
+      gv[k] = fact ? w - m : m;
+    }, [&](uint32_t e, int k) { x[e] = gv[k]; });
+    __syncthreads();
+    if (fact) states(std::true_type{});
+    // ---- the parameter; the momentum into x ----
+    {
+      CAME8_GLOBAL PS* p = gbl(static_cast<PS*>(t.p));
+      float po[U];
+      if (fact) {
+        small_each<NT, U>(N, R, C, [&](uint32_t e, int k) {
+          gv[k] = TG::load(g[e]);
+          po[k] = TP::load(p[e]);
+          mo[k] = f32 ? m32[e] : m_q8(e);
+        }, [&](int row, int col, int k) {
+          gv[k] = m_new(((fac[row] * fac[R + col]) * gv[k]) / clip, mo[k]);
+          po[k] = param_update<TP>(po[k], (stv[row] * stv[R + col]) * gv[k], hp);
+        }, [&](uint32_t e, int k) {
+          p[e] = TP::store(po[k]);
+          x[e] = gv[k];
+        });
+      } else {
+        small_each<NT, U>(N, 1, N, [&](uint32_t e, int k) {
+          po[k] = TP::load(p[e]);
+          gv[k] = x[e];
+        }, [&](int, int, int k) { po[k] = param_update<TP>(po[k], gv[k], hp); }, [&](uint32_t e, int k) { p[e] = TP::store(po[k]); });
+      }
+    }
+    __syncthreads();
+    if (f32) {
+      for (int e = tid; e < N; e += NT) st_m(t)[e] = x[e];
+    } else {
+      small_quant<true, NW>(x, N, hp.B, t.mq, t.ma);
+    }
+    if (!fact) {  // the second moment, formed again from the old one
+      __syncthreads();
+      small_each<NT, U>(N, 1, N, load_v, [&](int, int, int k) { gv[k] = vec_v_from(gv[k], vo[k], hp); }, [&](uint32_t e, int k) {
+        if (f32) st_sq_row(t)[e] = gv[k];
+        else x[e] = gv[k];
+      });
+      __syncthreads();
+      if (!f32) small_quant<false, NW>(x, N, hp.B, t.rq, t.ra);
+    }
+    __syncthreads();  // the LDS is used again
+  }
 }
 
 }  // namespace came8

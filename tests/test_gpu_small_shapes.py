@@ -34,6 +34,21 @@ def test_tiny_matrices(dtype, block, exact_norm):
     _run(came_amd.CAME8bitFull, TINY, dtype, block, exact_norm, heavy=block == 256, seed=71)
 
 
+# one workgroup's steps: a row, a column, both sizes' edges (4096 and 32768 elements, 2560 rows and columns) and just
+# past them, rows of fewer and more columns than threads, lengths with every tail of the norm's chains
+SMALL = [(1,), (7,), (12,), (4095,), (4096,), (4099,), (32768,), (32769,), (1, 1), (1, 300), (300, 1), (5, 8), (96, 200),
+         (16, 1280), (1280, 16), (2560, 12), (12, 2548), (13, 2548), (64, 64), (65, 63), (181, 181), (256, 128),
+         (129, 255), (31, 1057), (1, 32767), (1, 4, 1000), (3, 40, 60)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block", [64, 100, 256, 4096])
+@pytest.mark.parametrize("exact_norm", [False, True])
+def test_small_tensors(dtype, block, exact_norm):
+    heavy = block == 64 and dtype != torch.float16
+    _run(came_amd.CAME8bitFull, SMALL, dtype, block, exact_norm, heavy=heavy, seed=91)
+
+
 @pytest.mark.parametrize("cls", ["CAME8bitFull", "CAMECUDA"])
 def test_unaligned_buffers_match_aligned_ones(cls):
     """The vector forms and the ones that buffers off 16-byte boundaries take: the same step.  Sums may be ordered
