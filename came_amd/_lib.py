@@ -7,11 +7,13 @@ fails to load, every entry point that needs it raises ``RuntimeError``.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libcame8.so")
+HOST_PATH = os.path.join(HERE, "lib", "came8_host.so")  # csrc/came8_host.cpp
 
 CAME8_F32, CAME8_BF16, CAME8_F16 = 0, 1, 2
 CAME8_OK, CAME8_EINVAL, CAME8_ESPACE, CAME8_EHIP = 0, -1, -2, -3
@@ -103,6 +105,7 @@ class Came8PhaseStat(ctypes.Structure):
 
 
 _lib = None
+_host = None
 _lock = threading.Lock()
 _tag_lock = threading.Lock()
 _next_tag = [0]
@@ -165,6 +168,23 @@ def load(path: str | None = None) -> ctypes.CDLL:
             raise RuntimeError(f"came_amd: {p} has ABI {lib.came8_abi_version()}, expected {ABI_VERSION}")
         _lib = lib
         return lib
+
+
+def host():
+    """The native descriptor gathering (csrc/came8_host.cpp), loaded once; RuntimeError if it is missing."""
+    global _host
+    if _host is None:
+        with _lock:
+            if _host is None:
+                if not os.path.exists(HOST_PATH):
+                    raise RuntimeError(
+                        f"came_amd: {HOST_PATH} not found; build it with `python -c \"import came_amd.build as b; b.build()\"`"
+                    )
+                spec = importlib.util.spec_from_file_location("came8_host", HOST_PATH)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                _host = mod
+    return _host
 
 
 def check(rc: int, what: str) -> None:

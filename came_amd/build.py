@@ -22,6 +22,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "lib")
 OUT = os.path.join(OUT_DIR, "libcame8.so")
+HOST_OUT = os.path.join(OUT_DIR, "came8_host.so")  # descriptor gathering for the optimizers, host code only
 ARCH = os.environ.get("CAME8_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [
@@ -51,6 +52,20 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
+def host_cmd(out: str) -> list[str]:
+    """The compiler line of the host extension: plain C++ against torch's and Python's headers."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    inc = [f for i in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"]) for f in ("-isystem", i)]
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, "-o", out,
+            os.path.join(CSRC, "came8_host.cpp"), *(f"-L{p}" for p in cpp_extension.library_paths()),
+            "-ltorch_python", "-ltorch_cpu", "-lc10"]
+
+
 def _run(cmd: list[str]) -> tuple[int, str]:
     res = subprocess.run(cmd, capture_output=True, text=True)
     noise = "packed-fp32-ops"  # hipcc's host pass does not know the device feature
@@ -70,14 +85,16 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
         obj = os.path.join(OUT_DIR, f"{name}.o")
         objs.append(obj)
         cmds.append([cc, *HIPCC_FLAGS, *defs, *inc, "-c", "-o", obj, os.path.join(CSRC, src)])
+    host_tmp = HOST_OUT + ".tmp"
+    cmds.append(host_cmd(host_tmp))
     jobs = jobs or min(len(cmds), os.cpu_count() or 1)
     if verbose:
         print(f"[came_amd.build] {len(cmds)} units, {jobs} parallel: {' '.join(cmds[0])}", flush=True)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         results = list(ex.map(_run, cmds))
-    for (name, _, _), (rc, errs) in zip(UNITS, results):
+    for name, (rc, errs) in zip([u[0] for u in UNITS] + ["came8_host"], results):
         if rc != 0:
-            raise RuntimeError(f"hipcc failed on {name} ({rc}):\n{errs}")
+            raise RuntimeError(f"compiling {name} failed ({rc}):\n{errs}")
         if verbose and errs.strip():
             print(errs, file=sys.stderr)
     tmp = OUT + ".tmp"
@@ -87,6 +104,7 @@ def build(verbose: bool = True, jobs: int | None = None) -> str:
     for o in objs:
         os.remove(o)
     os.replace(tmp, OUT)
+    os.replace(host_tmp, HOST_OUT)
     return OUT
 
 

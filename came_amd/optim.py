@@ -367,7 +367,6 @@ class _Came8Base(torch.optim.Optimizer):
         by_device: dict = defaultdict(list)
         for p in params:
             by_device[p.device].append(p)
-        lib = _lib.load()
         for device, plist in by_device.items():
             items = []
             for p in plist:
@@ -381,16 +380,44 @@ class _Came8Base(torch.optim.Optimizer):
                 continue
             n = len(items)
             descs, keep, copyback = self._descriptors(items, block_size)
-            ws, tag = self._workspace(group, device, descs, n, block_size)
-            with torch.cuda.device(device):
-                stream = torch.cuda.current_stream(device).cuda_stream
-                _lib.check(lib.came8_step(descs, n, ctypes.byref(hp), ws.data_ptr(), ws.numel(), tag, stream),
-                           "came8_step")
+            self._launch(group, device, descs, n, hp, block_size)
             if plan_only:
                 continue
             self.__dict__.setdefault("_came8_last_step", {})[(device, id(group))] = [p for p, _, _ in items]
             for p, pd in copyback:
                 p.data.copy_(pd)
+
+    def _launch(self, group: dict, device: torch.device, descs, n: int, hp, block_size: int) -> None:
+        lib = _lib.load()
+        ws, tag = self._workspace(group, device, descs, n, block_size)
+        with torch.cuda.device(device):
+            stream = torch.cuda.current_stream(device).cuda_stream
+            _lib.check(lib.came8_step(descs, n, ctypes.byref(hp), ws.data_ptr(), ws.numel(), tag, stream),
+                       "came8_step")
+
+    def _step_group_native(self, group: dict) -> int | None:
+        """The group's step with its descriptors gathered natively: the number of tensors stepped, or None
+        when the group is not the plain case (csrc/came8_host.cpp) and the Python has to take it."""
+        params = group["params"]
+        if self._STATE_KIND not in (_lib.CAME8_STATE_Q8, _lib.CAME8_STATE_FP32) or self._rounds_fp16():
+            return None
+        if type(params) is not list or not params:
+            return None
+        block_size = self._group_block_size(group)
+        descs = (_lib.Came8Tensor * len(params))()
+        hp = self._group_hparams(group)
+        used = _lib.host().gather(params, self.state, ctypes.addressof(descs), len(params), self._STATE_KIND, block_size)
+        if used is None:
+            return None
+        if used:
+            device = used[0].device
+            self._launch(group, device, descs, len(used), hp, block_size)
+            self.__dict__.setdefault("_came8_last_step", {})[(device, id(group))] = used
+        return len(used)
+
+    def _rounds_fp16(self) -> bool:
+        """Whether some 1-D tensor may take the fp16-rounded update (_fp16_update_tensors)."""
+        return bool(getattr(self, "cuda_nonfactored_use_fp16_update", False))
 
     def _fp16_update_tensors(self, items: list, block_size: int) -> list:
         """Which of the (param, state, grad) items take the reference's fp16-update rounding of the 1-D update
@@ -459,6 +486,10 @@ class _Came8Base(torch.optim.Optimizer):
         t0 = time.perf_counter()
         count = 0
         for group in self.param_groups:
+            stepped = self._step_group_native(group)
+            if stepped is not None:
+                count += stepped
+                continue
             params = []
             for p in group["params"]:
                 if p.grad is None:
@@ -694,6 +725,9 @@ class CAME8bit(CAME8bitFull):
     @classmethod
     def _experimental_cuda_tuning_overrides(cls, **kwargs) -> tuple[str, ...]:
         return tuple(k for k, default in cls.EXPERIMENTAL_CUDA_TUNING_DEFAULTS.items() if kwargs[k] != default)
+
+    def _rounds_fp16(self) -> bool:
+        return super()._rounds_fp16() or (self.prefer_cuda_1d_multitensor_fast_path and self.cuda_1d_batched_use_fp16_update)
 
     @torch.no_grad()
     def _fp16_update_tensors(self, items: list, block_size: int) -> list:
