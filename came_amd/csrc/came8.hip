@@ -121,7 +121,7 @@ struct Plan {
   std::map<TypeKey, WorkList> generic;   // P3 / B for other block sizes (per quantisation block)
   // the clip's norm in the reference's order (came8_norm.h)
   WorkList nest_w;                       // unit estimates, a workgroup per row band (matrices >= 256 wide)
-  WorkList nest_n;                       // unit estimates, a thread per unit (per 256 units)
+  WorkList nest_n;                       // unit estimates, kEstLanes lanes per unit (per kEstUnits units)
   std::map<int, WorkList> nseg2d;        // segment records of matrices, runs of nrun segments, by 3 * grad type + form
   std::map<int, WorkList> nseg;          // the other segments' records, by 3 * grad type + chunk form
   WorkList nbsum;                        // the chains' sums per block of segments (one item per block)
@@ -570,7 +570,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
       d.nrun = d.nseg0 >= 256 * int64_t(kNormRunSegs) ? kNormRunSegs : (d.nseg0 >= 128 * int64_t(kNormRunSegs) ? 32 : 16);
       const int64_t nbase = t.factored ? d.P * d.nbands : d.nclip;
       if (tiny_matrix(t, false)) d.ngrp = tiny_group(d.P);
-      // the thread-per-unit estimate groups single-band matrices and tiles into at most kNormMaxUnits units
+      // the narrow estimate groups single-band matrices and tiles into at most kNormMaxUnits units
       else if (!norm_est_wide(t, d) && (!t.factored || d.nbands == 1)) d.ngrp = ceil_div(nbase, kNormMaxUnits);
       d.nunit = ceil_div(nbase, d.ngrp);
       o.nest = take(size_t(d.nunit + 1) * 4);
@@ -719,7 +719,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     // one segment needs no estimates, records or rebuild.
     if (d.nseg > 1) {
       if (norm_est_wide(t, d)) add_item(plan.nest_w, i, d.nunit);
-      else if (!tiny_matrix(t, false)) add_item(plan.nest_n, i, ceil_div(d.nunit, int64_t(kThreads)));
+      else if (!tiny_matrix(t, false)) add_item(plan.nest_n, i, ceil_div(d.nunit, int64_t(kEstUnits)));
       // the vector forms need rows of whole aligned 8-element chunks and 32-bit flat indices; matrices
       // (prefix 1) up to kNormLdsCols wide take runs of segments with their column factors in LDS
       const bool vec = t.factored && d.idx32 && reinterpret_cast<uintptr_t>(t.grad) % 16 == 0;

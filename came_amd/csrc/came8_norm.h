@@ -135,11 +135,16 @@ constexpr uint32_t kNormFull = 1u << 24;
 //   rm * (sum_i e_i / R_i) * (sum_j c_j^2 U_j) / (sum_j U_j),   e_i = sum_j g_ij^2,
 // exact when the rows' profiles agree (Gaussian rows: ~1e-5 relative per band) and a few percent off
 // on heavy-tailed rows; k_norm_fix rebuilds the records of a chain that the estimate misleads.
-__device__ __forceinline__ float norm_unit_rm(const DevTensor& t, int64_t u) {
-  return matrix_row_mean(t, t.rsum, u / t.nbands, t.nbands);
+// WIDE: a workgroup per unit (matrices of at least 256 columns); otherwise kEstLanes lanes per unit: a thread per unit
+// read its row of partials serially, four workgroups a launch for a thousand bands, bound by one load after the other
+// (bands of four matrices of 24 to 200 columns among 30 tensors: 39 -> 11 us).
+constexpr int kEstLanes = 16, kEstUnits = kThreads / kEstLanes;  // lanes of a unit, units of a workgroup
+template <typename T>
+__device__ __forceinline__ T est_lanes_sum(T v) {
+#pragma unroll
+  for (int o = kEstLanes / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kEstLanes);
+  return v;
 }
-
-// WIDE: a workgroup per unit (matrices of at least 256 columns); otherwise a thread per unit.
 template <bool WIDE>
 __global__ __launch_bounds__(kThreads) void k_norm_est(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
                                                        const int64_t* __restrict__ wstart, int ntens, Hp hp) {
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void k_norm_est(const DevTensor* __restri
         acc[0] = fmaf(cf[j] * cf[j], Up[j], acc[0]);
         accu[0] += Up[j];
       }
-      // the matrix's mean row state (norm_unit_rm's): the workgroup sums the band sums, thread k over
+      // the matrix's mean row state: the workgroup sums the band sums, thread k over
       // sums k, k + 256, ... (one round of loads, not one thread's chain after the reductions)
       double rp = 0.0;
       for (int64_t k = tid; k < t.nbands; k += kThreads) rp += double(t.rsum[m * t.nbands + k]);
@@ -203,28 +208,36 @@ __global__ __launch_bounds__(kThreads) void k_norm_est(const DevTensor* __restri
       }
       __syncthreads();
     } else {
-      const int64_t u = (w - wstart[slot]) * kThreads + tid;
+      const int64_t u = (w - wstart[slot]) * kEstUnits + tid / kEstLanes;
+      const int l = tid % kEstLanes;
       if (u >= t.nunit) continue;
       // the unit's ngrp base units: row bands, or (ngrp > 1) whole single-band matrices, or tiles
       const int64_t nbase = t.factored ? t.P * t.nbands : t.nclip;
       const int64_t b0 = u * t.ngrp, b1 = min(nbase, b0 + t.ngrp);
       float e = 0.0f;
-      for (int64_t b = b0; b < b1; ++b) {
-        if (t.factored) {  // a band pass of the default mode: the band's profile of g^2
+      if (t.factored) {  // a band pass of the default mode: the band's profile of g^2
+        for (int64_t b = b0; b < b1; ++b) {
           const int64_t m = b / t.nbands;
           const float* __restrict__ Up = t.partU + b * t.C;
           const float* __restrict__ cf = t.cfac + m * t.C;
           float s = 0.0f, su = 0.0f;
-          for (int64_t j = 0; j < t.C; ++j) {
+#pragma unroll 4
+          for (int64_t j = l; j < t.C; j += kEstLanes) {
             s = fmaf(cf[j] * cf[j], Up[j], s);
             su += Up[j];
           }
-          e += su > 0.0f ? norm_unit_rm(t, b) * t.esum[b] * (s / su) : 0.0f;
-        } else {
-          e += float(t.clip_part[b]);
+          double rp = 0.0;  // the matrix's mean row state
+          for (int64_t k = l; k < t.nbands; k += kEstLanes) rp += double(t.rsum[m * t.nbands + k]);
+          s = est_lanes_sum(s);
+          su = est_lanes_sum(su);
+          rp = est_lanes_sum(rp);
+          e += su > 0.0f ? row_mean_of_sum(t, rp) * t.esum[b] * (s / su) : 0.0f;
         }
+      } else {
+        for (int64_t b = b0 + l; b < b1; b += kEstLanes) e += float(t.clip_part[b]);
+        e = est_lanes_sum(e);
       }
-      t.nest[u] = e;
+      if (l == 0) t.nest[u] = e;
     }
   }
 }
