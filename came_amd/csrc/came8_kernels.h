@@ -20,6 +20,9 @@
 //       parameter write, int8 requantisation of m.
 //   B   1-D tensors: v, u/clip, m, parameter write, int8 + uint8 requantisation.
 //
+// Matrices of at most 64 elements form their factors inside P1 and P2 (k_tiny_pass1, k_tiny_pass2), and a call
+// whose tensors are all small runs whole in one launch (k_small_step in came8_norm.h).
+//
 // The arithmetic of every element follows the reference's CPU path
 // (came_pytorch/CAME8bitFull.py:1006-1075) operation for operation, with the
 // same roundings (fused multiply-add where torch's CPU kernels fuse, IEEE

@@ -14,13 +14,11 @@
 // and fma(x, x, s) = (m + n) * 2^(E-23) with n = round(x^2 * 2^(23-E)), provided m + n < 2^24 and
 // x^2 * 2^(23-E) is not a half-integer: the exact sum then lies strictly inside the binade, whose
 // floats are exactly the multiples of 2^(E-23).  So inside a binade the chain is an integer sum of
-// per-element increments that do not depend on s.  Elements whose increment is not determined this
-// way are "special": the rounded square x*x is a half-integer after scaling (the true square may be
-// a tie, whose rounding depends on m's parity), or x*x is infinite or NaN; an element whose increment
-// takes the chain out of the binade ends the run of known increments.  (When the rounded square is
-// not a half-integer, the true square rounds the same way: its distance to hi = RN(x*x) is at most
-// half an ulp of hi, less than the distance from hi to any half-integer, for every binade above the
-// subnormal one, whose half-integers lie on hi's grid.)
+// per-element increments that do not depend on s.  An element whose increment is not determined this
+// way is "special": its square is a half-integer after scaling (a tie, whose rounding depends on m's
+// parity), or infinite or NaN; an element whose increment takes the chain out of the binade ends the
+// run of known increments.  The increments are formed by the same fused multiply-add, into two sums
+// one unit apart (norm_base's comment says how they show a special element).
 //
 //   k_norm_est               an estimate of each chain's value along the tensor, from sums the step
 //                            has already formed (per row band: rm * sum_j c_j^2 * sum_i g_ij^2 / R_i;
@@ -28,8 +26,8 @@
 //                            before a segment themselves (norm_unit_prefix).
 //   k_norm_seg               one workgroup per segment of kNormSegElems elements (512 per chain):
 //                            per chain, the candidate binade Ea of the estimate (and Ea + 1 near a
-//                            binade edge), the integer sums of the increments under each, whether
-//                            the segment holds special elements, and whether it holds a NaN; and
+//                            binade edge), the integer sums of the increments under each, or that
+//                            the segment holds special elements or leaves the binade; and
 //                            the chain's fp32 sum of the segment's rounded squares.
 //   k_norm_bsum, k_norm_fix  each chain's own estimate (the prefix of its segment sums), and records
 //                            rebuilt under that estimate's binades where the tensor-wide estimate
@@ -53,11 +51,6 @@
 // addition on the chain; everything else is exact integer arithmetic, so the result equals the
 // serial chain bit for bit whatever the estimates were (they only decide how many segments are
 // replayed).
-//
-// The subnormal binade E = -126 (unit 2^-149, which is also the spacing of subnormal squares) has
-// one more special element: |x| = 2^-75, whose square 2^-150 is half a unit (a tie) but rounds to 0
-// as x * x.  (For |x| = k * 2^-75 with odd k > 1 the square rounds to a nonzero multiple of the
-// unit, which is special there already.)
 #pragma once
 
 #include "came8_kernels.h"
