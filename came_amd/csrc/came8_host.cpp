@@ -135,6 +135,7 @@ PyObject* gather(PyObject*, PyObject* args) {
   int kind;
   if (!PyArg_ParseTuple(args, "O!O!KLiL", &PyList_Type, &params, &PyDict_Type, &state, &addr, &cap, &kind, &block))
     return nullptr;
+  if (block < 1) Py_RETURN_NONE;  // the blocks are counted by a division; the Python raises the error
   try {
     came8_tensor* out = reinterpret_cast<came8_tensor*>(static_cast<uintptr_t>(addr));
     const Py_ssize_t n = PyList_GET_SIZE(params);

@@ -27,6 +27,31 @@ def test_cpu_parameters_are_left_to_the_python():
     assert _gather(opt, [p])[0] == []
 
 
+@pytest.mark.parametrize("block", [0, -1])
+def test_block_sizes_without_blocks_are_left_to_the_python(block):
+    """Before any tensor is looked at, so also for a group without gradients."""
+    p = torch.nn.Parameter(torch.zeros(4, 4))
+    opt = came_amd.CAME8bit([p], lr=1e-3)
+    opt.param_groups[0]["block_size"] = block
+    assert _gather(opt, [p])[0] is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [0, -1])
+def test_block_sizes_without_blocks_raise(block):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    p = torch.nn.Parameter(torch.zeros(4, 6, device="cuda"))
+    p.grad = torch.ones_like(p)
+    opt = came_amd.CAME8bit([p], lr=1e-3)
+    opt.step()  # with a state, which the native gathering would otherwise take
+    before = p.detach().clone()
+    opt.param_groups[0]["block_size"] = block
+    with pytest.raises(ValueError, match="block_size must be > 0"):
+        opt.step()
+    assert torch.equal(p.detach(), before) and opt.state[p]["step"] == 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("cls", ["CAME8bit", "CAME8bitFull", "CAME8bitMemory", "CAMECUDA"])
 def test_same_descriptors_as_the_python(cls):
