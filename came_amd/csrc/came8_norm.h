@@ -1498,7 +1498,7 @@ __device__ __forceinline__ void small_sums(Val val, int R, int C, double* dsum, 
 template <bool SIGNED, int NW>
 __device__ __forceinline__ void small_quant(const float* x, int n, int B, void* q, float* a) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int nb = (n + B - 1) / B;
+  const int nb = (n - 1) / B + 1;  // n >= 1; n + B may be past 2^31
   CAME8_GLOBAL uint8_t* qb = gbl(static_cast<uint8_t*>(q));
 #pragma unroll 1
   for (int blk = wid; blk < nb; blk += NW) {

@@ -83,3 +83,24 @@ def test_unaligned_buffers_match_aligned_ones(cls):
                 assert torch.allclose(w, v, rtol=1e-4, atol=1e-5 * v.abs().max().item()), (s, k)
             else:
                 assert (w.int() - v.int()).abs().max() <= 1, (s, k)
+
+
+@pytest.mark.parametrize("cls", ["CAME8bit", "CAME8bitMemory"])
+def test_block_sizes_far_past_the_tensors(cls):
+    """Every block size from the largest state's length up is one block a state: the same bits for all of them, also where
+    a length and a block size together pass 2^31."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    out = []
+    for block in (32768, 2**31 - 1000, 2**31 - 1):
+        gen = torch.Generator().manual_seed(3)
+        ps = []
+        for s in [(5, 7), (96, 200), (10,), (32768,), (1, 2048)]:
+            ps.append(torch.nn.Parameter((torch.randn(s, generator=gen) * 0.02).cuda()))
+            ps[-1].grad = (torch.randn(s, generator=gen) * 1e-3).cuda()
+        opt = getattr(came_amd, cls)(ps, block_size=block, **HP)
+        for _ in range(2):
+            opt.step()
+        out.append([p.detach() for p in ps] + [v for p in ps for v in opt.state[p].values() if isinstance(v, torch.Tensor)])
+    for got in out[1:]:
+        assert len(got) == len(out[0]) and all(torch.equal(a, b) for a, b in zip(got, out[0]))
