@@ -1,9 +1,12 @@
-"""Edge shapes of the thread-per-matrix passes and of the kernels for small and narrow tensors, each step teacher-forced
-against the oracle under the tolerances of test_gpu_parity.py, and steps over unaligned buffers against aligned ones."""
+"""Edge shapes of the thread-per-matrix passes, of the kernels for small and narrow tensors and of the one-workgroup step,
+each step teacher-forced against the oracle under the tolerances of test_gpu_parity.py; the one-workgroup step against the
+passes, and steps over unaligned buffers against aligned ones."""
 import pytest
 import torch
 
 import came_amd
+from came_amd import _lib
+from oracle import came8_oracle as orc
 from tests import parity as P
 from tests.test_gpu_parity import _tight_step_check
 
@@ -34,8 +37,8 @@ def test_tiny_matrices(dtype, block, exact_norm):
     _run(came_amd.CAME8bitFull, TINY, dtype, block, exact_norm, heavy=block == 256, seed=71)
 
 
-# one workgroup's steps: a row, a column, both sizes' edges (4096 and 32768 elements, 2560 rows and columns) and just
-# past them, rows of fewer and more columns than threads, lengths with every tail of the norm's chains
+# Small and just larger tensors in one call: the larger ones take them all through the passes, with rows of fewer and more
+# columns than threads and lengths with every tail of the norm's chains.
 SMALL = [(1,), (7,), (12,), (4095,), (4096,), (4099,), (32768,), (32769,), (1, 1), (1, 300), (300, 1), (5, 8), (96, 200),
          (16, 1280), (1280, 16), (2560, 12), (12, 2548), (13, 2548), (64, 64), (65, 63), (181, 181), (256, 128),
          (129, 255), (31, 1057), (1, 32767), (1, 4, 1000), (3, 40, 60)]
@@ -47,6 +50,175 @@ SMALL = [(1,), (7,), (12,), (4095,), (4096,), (4099,), (32768,), (32769,), (1, 1
 def test_small_tensors(dtype, block, exact_norm):
     heavy = block == 64 and dtype != torch.float16
     _run(came_amd.CAME8bitFull, SMALL, dtype, block, exact_norm, heavy=heavy, seed=91)
+
+
+# One workgroup's steps.  SHORT takes 256 threads a tensor (up to 2048 elements), LONG 1024 (up to 32768 elements and 2560
+# rows and columns): a row, a column, both sizes' edges, rows of fewer and more columns than threads, and lengths with
+# every remainder of the norm's eight chains below and above their 16-element batches.
+SHORT = [(1,), (2,), (3,), (4,), (5,), (6,), (7,), (8,), (12,), (13,), (14,), (15,), (127,), (129,), (2041,), (2042,),
+         (2043,), (2044,), (2045,), (2046,), (2047,), (2048,), (1, 1), (1, 300), (300, 1), (5, 8), (64, 32), (45, 45),
+         (2, 1024), (1024, 2), (1, 2048), (2048, 1), (1, 4, 500)]
+LONG = [(2049,), (4095,), (4096,), (4099,), (32761,), (32766,), (32767,), (32768,), (96, 200), (16, 1280), (1280, 16),
+        (2547, 12), (12, 2548), (13, 2520), (64, 64), (65, 63), (181, 181), (256, 128), (127, 258), (31, 1057),
+        (1, 2559), (2559, 1), (1, 40, 800), (1, 1, 16, 2032)]
+# just past an edge, each of which takes a whole call through the passes
+PAST = [(32769,), (129, 255), (13, 2548), (1, 2560), (2560, 1), (3, 40, 60)]
+
+
+def _phases(step):
+    """The kernels that step() launched, by name."""
+    _lib.profile_enable(True)
+    try:
+        _lib.profile_read(reset=True)
+        step()
+        torch.cuda.synchronize()
+        return {k for k, v in _lib.profile_read(reset=True).items() if v[0]}
+    finally:
+        _lib.profile_enable(False)
+
+
+def _optimizer(cls, shapes, dtype=torch.float32, gdtype=None, offset=0, seed=5, std=1e-3, **kw):
+    """An optimizer over tensors `offset` elements into their buffers."""
+    gen = torch.Generator().manual_seed(seed)
+    ps = []
+    for s in shapes:
+        n = torch.Size(s).numel()
+        p = torch.empty(n + offset, device="cuda", dtype=dtype)[offset:].view(s)
+        g = torch.empty(n + offset, device="cuda", dtype=gdtype or dtype)[offset:].view(s)
+        p.copy_(torch.randn(s, generator=gen) * 0.02)
+        g.copy_(torch.randn(s, generator=gen) * std)
+        q = torch.nn.Parameter(p)
+        if gdtype is not None:
+            q.grad_dtype = gdtype
+        q.grad = g
+        ps.append(q)
+    return ps, getattr(came_amd, cls)(ps, **{**HP, **kw})
+
+
+@pytest.mark.parametrize("shapes", [SHORT, LONG, SHORT + LONG], ids=["short", "long", "both"])
+@pytest.mark.parametrize("cls", ["CAME8bitFull", "CAMECUDA"])
+def test_calls_of_small_tensors_take_one_launch(shapes, cls):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    _, opt = _optimizer(cls, shapes)
+    assert _phases(opt.step) == {"small_step"}
+    for s in PAST:
+        _, opt = _optimizer(cls, SHORT[:3] + [s])
+        ran = _phases(opt.step)
+        assert "small_step" not in ran and ran, s
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("block", [64, 100, 256, 4096])
+@pytest.mark.parametrize("exact_norm", [False, True])
+@pytest.mark.parametrize("shapes", [SHORT, LONG], ids=["short", "long"])
+def test_one_workgroup_steps(shapes, dtype, block, exact_norm):
+    heavy = block == 64 and dtype != torch.float16
+    _run(came_amd.CAME8bitFull, shapes, dtype, block, exact_norm, heavy=heavy, seed=91)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("block", [256, 100])
+def test_small_vectors_with_the_fp16_rounded_update(dtype, block):
+    """Teacher-forced against the oracle's fp16_update branch, as test_gpu_fp16_update.py runs it on calls that hold a
+    large tensor."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    shapes = [s for s in SHORT + LONG if len(s) == 1]
+    params = P.make_params(shapes, dtype, seed=block)
+    gen = torch.Generator().manual_seed(block + 1)
+    hp = dict(HP, block_size=block)
+    ps = [torch.nn.Parameter(p.cuda()) for p in params]
+    opt = came_amd.CAME8bitFull(ps, cuda_nonfactored_use_fp16_update=True, **hp)
+    sts = [orc.init_full8bit_state(p.shape, block) for p in params]
+    check = _tight_step_check(f"small fp16 update {dtype} B={block}", block=block)
+    for step in range(2):
+        with torch.no_grad():
+            for p, r, st in zip(ps, params, sts):
+                p.data.copy_(r)
+                for k in P.STATE_KEYS:
+                    if len(opt.state[p]) and k in st:
+                        opt.state[p][k].copy_(st[k])
+        grads = [P.heavy_grad(gen, s, dtype) for s in shapes]
+        for p, g in zip(ps, grads):
+            p.grad = g.cuda()
+        assert _phases(opt.step) == {"small_step"}
+        for i, (r, g, st) in enumerate(zip(params, grads, sts)):
+            before, cap = r.double(), {}
+            orc.full8bit_step(r, g, st, capture=cap, fp16_update=True, **P.oracle_hp(hp))
+            check(step + 1, i, ps[i].data, r, opt.state[ps[i]], st, (r.double() - before).abs(), cap)
+
+
+# the one launch against the passes, which one large tensor more in the call brings about: every class, pair of types,
+# alignment, block size and mode that both take
+ROUTES = [dict(cls="CAME8bitFull"), dict(cls="CAME8bitFull", block_size=100), dict(cls="CAME8bitFull", block_size=2048),
+          dict(cls="CAME8bitFull", offset=1), dict(cls="CAME8bitFull", exact_norm=True),
+          dict(cls="CAME8bitFull", cuda_nonfactored_use_fp16_update=True, block_size=64),
+          dict(cls="CAME8bitFull", dtype=torch.bfloat16, offset=3), dict(cls="CAME8bitFull", dtype=torch.float16),
+          dict(cls="CAME8bitFull", dtype=torch.bfloat16, gdtype=torch.float32),
+          dict(cls="CAME8bitFull", dtype=torch.float32, gdtype=torch.float16),
+          dict(cls="CAME8bitMemory", betas=(0.9, 0.95, 0.995), weight_decay=0.0), dict(cls="CAME8bit", clip_threshold=0.25),
+          dict(cls="CAMECUDA"), dict(cls="CAMECUDA", offset=1, exact_norm=True), dict(cls="CAMECUDA", dtype=torch.bfloat16)]
+
+
+@pytest.mark.parametrize("route", ROUTES, ids=lambda r: "-".join(str(v) for v in r.values()))
+def test_one_launch_matches_the_passes(route):
+    """Sums may be ordered otherwise, hence the tolerances of the parity tests (codes one apart, 1e-5 of parameters and
+    scales); a 16-bit parameter may round to its neighbour."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    route = dict(route)
+    exact = route.pop("exact_norm", False)
+    cls = route.pop("cls")
+    shapes = SHORT + LONG
+    out = []
+    for more in ([], [(300, 200)]):
+        ps, opt = _optimizer(cls, shapes + more, **route)
+        opt.exact_norm = exact
+        ran = _phases(opt.step)
+        assert (ran == {"small_step"}) == (not more)
+        out.append((ps, [opt.state[p] for p in ps]))
+    _same_steps(out, shapes, {torch.float32: 0.0, torch.bfloat16: 2**-7, torch.float16: 2**-10}[out[0][0][0].dtype])
+
+
+def _same_steps(out, shapes, ulp=0.0):
+    for i, s in enumerate(shapes):
+        a, b = out[0][0][i].data.double(), out[1][0][i].data.double()
+        assert ((a - b).abs() <= (1e-5 + ulp) * b.abs() + 2e-7 + 1e-3 * HP["lr"]).all(), s
+        for k, v in out[1][1][i].items():
+            if not isinstance(v, torch.Tensor) or v.numel() == 0:
+                continue
+            w = out[0][1][i][k]
+            if v.dtype.is_floating_point:
+                assert torch.allclose(w, v, rtol=1e-4, atol=1e-5 * v.abs().max().item()), (s, k)
+            else:
+                assert (w.int() - v.int()).abs().max() <= 1, (s, k)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("cls", ["CAME8bitFull", "CAMECUDA"])
+def test_non_finite_gradients_match_the_passes(cls, bad):
+    """One infinite or NaN gradient in each of some tensors: the same parameters, scales and fp32 states come out NaN,
+    infinite and finite as from the passes, and the other tensors step bit for bit as without it."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    shapes = [(9,), (2048,), (4099,), (5, 8), (96, 200), (1, 300), (64, 32)]
+    hit = (1, 2, 3, 4)
+    out = []
+    for more, where in (([], hit), ([(300, 200)], hit), ([], ())):
+        ps, opt = _optimizer(cls, shapes + more)
+        for i in where:
+            ps[i].grad.view(-1)[7] = bad
+        ran = _phases(opt.step)
+        assert (ran == {"small_step"}) == (not more)
+        out.append([[p.data] + [v for v in opt.state[p].values() if isinstance(v, torch.Tensor) and v.dtype == torch.float32]
+                    for p in ps[: len(shapes)]])
+    for i, s in enumerate(shapes):
+        for a, b, c in zip(*(o[i] for o in out)):
+            assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.isinf(), b.isinf()), s
+            fin = a.isfinite()
+            assert torch.allclose(a[fin], b[fin], rtol=1e-4, atol=1e-6), s
+            assert i in hit or torch.equal(a, c), s
 
 
 @pytest.mark.parametrize("cls", ["CAME8bitFull", "CAMECUDA"])
