@@ -113,6 +113,7 @@ struct Plan {
   WorkList tinyq;                        // their states' codes (per four state blocks)
   // small tensors, a workgroup each for the whole step, by types: up to kSmallElems elements, and larger ones
   std::map<TypeKey, WorkList> smallS, smallL;
+  bool small[2] = {false, false};        // [exact clip]: those lists are the step, not the passes (small_call)
   std::map<TypeKey, WorkList> upd;       // P3, tile form (fast block sizes)
   std::map<TypeKey, WorkList> updb;      // P3, band form
   std::map<TypeKey, WorkList> vecB;      // 1-D pass B (fast block sizes)
@@ -245,13 +246,52 @@ bool small_tensor(const came8_tensor& t) {
   return !t.factored || t.rows + t.cols <= kSmallStates;
 }
 
-// The tensors take k_small_step when all of them can: beside larger tensors they ride along in launches that are made
-// anyway, at less than the 20 us that kernel takes for a vector of 2048 (292 tensors of a 24-layer model: 1965 us, 1986
-// with its 194 vectors in a launch of their own).
 bool all_small(const came8_tensor* ts, int32_t n) {
   for (int32_t i = 0; i < n; ++i)
     if (!small_tensor(ts[i])) return false;
   return true;
+}
+
+// Whether k_small_step takes a call, of tensors that all can (beside larger tensors they ride along in launches that are
+// made anyway, at less than the 20 us that kernel takes for a vector of 2048: 292 tensors of a 24-layer model 1965 us,
+// 1986 with its 194 vectors in a launch of their own).  It does unless the passes are faster (GPU time of both, us), which
+// they are nowhere with the block sizes that they have no vector forms for (800 of 16x2048 in blocks of 100: 1249 and 404):
+//   * A workgroup takes 60 to 100 us for a tensor near its limits, in a few tensors as in 256, and the passes little more
+//     than their launches: three for vectors, eight for matrices, twice as many for the default clip's chains.  kLone is
+//     the number of tensors past a size from which the launches' work outgrows that.  Exact clip: one vector of 4096 is
+//     20 in the passes and 19 here, one of 32768 21 and 60, 128 of them 61 and 72, 192 of them 82 and 77; one 16x1024 matrix 43
+//     and 42, one 16x2000 47 and 64, 64 of 16x2048 55 and 67, 96 of them 70 and 67.  Default clip: one vector of 24576
+//     68 and 59, one of 32768 68 and 75, 32 of them 81 and 77; matrices are faster here in any number.  fp32 states have
+//     no codes to write here and gain earlier.
+//   * Matrices of the 8-bit states in rows of whole 8-element chunks run at the passes' best rates, a few workgroups a CU,
+//     where a large one here fills a CU: past so many elements of them the passes win (kCrowd).  Default clip: 768 of
+//     16x2048 327 in the passes and 268 here, 896 of them 333 and 352, 1600 of them 661 and 731.  Exact clip: 512 of
+//     16x1024 102 and 93, 768 of them 129 and 138.  Odd rows, vectors and fp32 states were faster here in every number
+//     (2048 of 181x181 1235 and 974, 3200 of 16x2048 with fp32 states 1416 and 951).
+bool small_call(const came8_tensor* ts, int32_t n, int32_t B, bool exact) {
+  if (!fast_block(B)) return true;
+  constexpr int64_t kCrowd[2] = {768 * 32768, 10 << 20};
+  const int64_t crowd_size = exact ? 8192 : 16384;
+  bool mats = false, q8 = false;
+  for (int32_t i = 0; i < n; ++i) {
+    mats |= ts[i].factored != 0;
+    q8 |= ts[i].state_kind != CAME8_STATE_FP32;
+  }
+  int64_t size = kLargeElems, few = 0;  // fewer than `few` tensors above `size`: the passes
+  if (exact) {
+    size = mats ? 16384 : (q8 ? 4096 : 8192);
+    few = !q8 ? 64 : (mats ? 96 : 192);
+  } else if (!mats && q8) {
+    size = 28672;
+    few = 32;
+  }
+  int64_t lone = 0, crowd = 0;
+  for (int32_t i = 0; i < n; ++i) {
+    const int64_t N = ts[i].rows * ts[i].cols;
+    lone += N > size ? 1 : 0;
+    if (ts[i].factored && ts[i].state_kind != CAME8_STATE_FP32 && ts[i].cols % 8 == 0 && N > crowd_size) crowd += N;
+  }
+  return (lone == 0 || lone >= few) && crowd <= kCrowd[exact];
 }
 
 // Matrices per work item of those passes, and per unit of the clip-norm estimates (at most kNormMaxUnits of them)
@@ -402,12 +442,16 @@ std::vector<int> band_shrinks(const came8_tensor* ts, int32_t n, int32_t B) {
   return out;
 }
 
-int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan& plan) {
+// limit: the workspace's bytes.  A call of small tensors that the passes would be faster on has the passes' scratch too;
+// where that does not fit, k_small_step takes it in either mode (only_small).
+int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, size_t limit, Plan& plan, bool only_small = false) {
   if (n < 0) return fail(CAME8_EINVAL, "came8: n_tensors must be >= 0");
   if (n > 0 && ts == nullptr) return fail(CAME8_EINVAL, "came8: tensors is NULL");
   if (B <= 0) return fail(CAME8_EINVAL, "came8: block_size must be > 0, got " + std::to_string(B));
   plan.dev.assign(n, DevTensor{});
-  const bool small = all_small(ts, n);
+  const bool can_small = all_small(ts, n);
+  for (const bool exact : {false, true}) plan.small[exact] = can_small && (only_small || small_call(ts, n, B, exact));
+  const bool small = plan.small[false] && plan.small[true];  // no passes
   // --- scratch layout (after the plan blob; offsets relative to the scratch start) ---
   std::vector<size_t> scr_off(n, 0);
   size_t scr = 0;
@@ -661,10 +705,9 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
     const came8_tensor& t = ts[i];
     const DevTensor& d = plan.dev[i];
     const TypeKey tk{t.param_dtype, t.grad_dtype, d.fp32st};
-    if (small) {
+    if (plan.small[false] || plan.small[true])
       add_item((d.N <= kSmallElems ? plan.smallS : plan.smallL)[TypeKey{t.param_dtype, t.grad_dtype, 0}], i, 1);
-      continue;
-    }
+    if (small) continue;
     if (d.mode2d) {
       const BandShapeSel sel = band_variant(t, d.C, B, 1);
       add_item(plan.band2dw[BandKey{t.grad_dtype, sel.V, sel.K, sel.TPB, 0, sel.ua}], i, d.nbands);
@@ -788,6 +831,10 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, Plan
   off = plan.zero_off + kZeroBytes;
   plan.plan_bytes = align_up(off);
   plan.total_bytes = plan.plan_bytes + scr;
+  if (can_small && !small && plan.total_bytes > limit) {
+    plan = Plan{};
+    return build_plan(ts, n, B, ws_base, limit, plan, true);
+  }
 
   if (ws_base != nullptr) {
     char* scr_base = ws_base + plan.plan_bytes;
@@ -893,14 +940,15 @@ struct CacheEntry {
 };
 
 // The inputs a plan depends on, as bytes: the descriptor count, the block size, the workspace
-// address (the plan holds pointers into the workspace) and the descriptors themselves.
-std::vector<uint8_t> plan_inputs(const came8_tensor* ts, int32_t n, int32_t B, const void* ws) {
+// address (the plan holds pointers into the workspace) and size and the descriptors themselves.
+std::vector<uint8_t> plan_inputs(const came8_tensor* ts, int32_t n, int32_t B, const void* ws, size_t ws_bytes) {
   const size_t nb = size_t(std::max(n, 0)) * sizeof(came8_tensor);
-  std::vector<uint8_t> v(24 + sizeof(void*) + nb);
-  const int64_t head[3] = {n, B, current_device()};  // band sizes depend on the device
-  std::memcpy(v.data(), head, 24);
-  std::memcpy(v.data() + 24, &ws, sizeof(void*));
-  if (nb) std::memcpy(v.data() + 24 + sizeof(void*), ts, nb);
+  const int64_t head[4] = {n, B, current_device(), int64_t(ws_bytes)};  // band sizes depend on the device
+  constexpr size_t H = sizeof(head);
+  std::vector<uint8_t> v(H + sizeof(void*) + nb);
+  std::memcpy(v.data(), head, H);
+  std::memcpy(v.data() + H, &ws, sizeof(void*));
+  if (nb) std::memcpy(v.data() + H + sizeof(void*), ts, nb);
   return v;
 }
 std::mutex g_cache_mu;
@@ -1357,19 +1405,13 @@ int static_scratch(void** out) {
 // ===========================================================================
 // C ABI
 // ===========================================================================
-extern "C" {
-
-const char* came8_version(void) { return "came8-mi355x 0.1 (gfx950)"; }
-int came8_abi_version(void) { return CAME8_ABI_VERSION; }
-int came8_side_stream_count(void) { return int(side_queue_count()); }
-const char* came8_last_error(void) { return g_last_error.c_str(); }
-
-int came8_workspace_size(const came8_tensor* tensors, int32_t n_tensors, int32_t block_size, size_t* bytes) {
-  if (!bytes) return fail(CAME8_EINVAL, "came8_workspace_size: bytes is NULL");
-  // the size of a descriptor set already sized is remembered (callers ask on every step)
+namespace {
+// bytes of the plan of a workspace of `limit` bytes (build_plan); the size of a descriptor set already sized is
+// remembered (callers ask on every step)
+int plan_size(const came8_tensor* tensors, int32_t n_tensors, int32_t block_size, size_t limit, size_t* bytes) {
   static std::mutex mu;
   static std::map<std::vector<uint8_t>, size_t> sized;
-  const std::vector<uint8_t> k = plan_inputs(tensors, n_tensors, block_size, nullptr);
+  const std::vector<uint8_t> k = plan_inputs(tensors, n_tensors, block_size, nullptr, limit);
   {
     std::lock_guard<std::mutex> lk(mu);
     auto it = sized.find(k);
@@ -1379,13 +1421,26 @@ int came8_workspace_size(const came8_tensor* tensors, int32_t n_tensors, int32_t
     }
   }
   Plan plan;
-  const int rc = build_plan(tensors, n_tensors, block_size, nullptr, plan);
+  const int rc = build_plan(tensors, n_tensors, block_size, nullptr, limit, plan);
   if (rc != CAME8_OK) return rc;
   *bytes = plan.total_bytes;
   std::lock_guard<std::mutex> lk(mu);
   if (sized.size() >= 64) sized.clear();
   sized[k] = plan.total_bytes;
   return CAME8_OK;
+}
+}  // namespace
+
+extern "C" {
+
+const char* came8_version(void) { return "came8-mi355x 0.1 (gfx950)"; }
+int came8_abi_version(void) { return CAME8_ABI_VERSION; }
+int came8_side_stream_count(void) { return int(side_queue_count()); }
+const char* came8_last_error(void) { return g_last_error.c_str(); }
+
+int came8_workspace_size(const came8_tensor* tensors, int32_t n_tensors, int32_t block_size, size_t* bytes) {
+  if (!bytes) return fail(CAME8_EINVAL, "came8_workspace_size: bytes is NULL");
+  return plan_size(tensors, n_tensors, block_size, SIZE_MAX, bytes);
 }
 
 int came8_release_workspace(const void* workspace) {
@@ -1413,7 +1468,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
   int rc = CAME8_OK;
   const auto key = std::make_pair(static_cast<const void*>(workspace), workspace_tag);
   std::vector<uint8_t> inputs;
-  if (workspace_tag) inputs = plan_inputs(tensors, n_tensors, h.block_size, workspace);
+  if (workspace_tag) inputs = plan_inputs(tensors, n_tensors, h.block_size, workspace, workspace_bytes);
   std::shared_ptr<const Plan> cached;
   if (workspace_tag) {
     std::lock_guard<std::mutex> lk(g_cache_mu);
@@ -1433,7 +1488,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
       return fail(CAME8_EINVAL, "came8_step: the stream is capturing and no launch plan exists for these tensors and "
                                 "this workspace; run one step (or a CAME8_FLAG_PLAN_ONLY call) before capture");
     built = std::make_shared<Plan>();
-    rc = build_plan(tensors, n_tensors, h.block_size, static_cast<char*>(workspace), *built);
+    rc = build_plan(tensors, n_tensors, h.block_size, static_cast<char*>(workspace), workspace_bytes, *built);
     if (rc != CAME8_OK) return rc;
   }
   const Plan& plan = cached ? *cached : *built;
@@ -1571,23 +1626,26 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
   bool split = false;  // the long-chain group runs on the side stream (set by the clip-norm section)
 
   // ---- small tensors: the whole step ----
-  for (const bool large : {false, true}) {
-    for (auto& kv : large ? plan.smallL : plan.smallS) {
-      const WorkList& wl = kv.second;
-      SmallFn fn;
-      if (large) CAME8_TYPE_SWITCH2(k_small_step_L, kv.first.pdt, kv.first.gdt, fn);
-      else CAME8_TYPE_SWITCH2(k_small_step_S, kv.first.pdt, kv.first.gdt, fn);
-      const int nt = large ? kLargeThreads : kSmallThreads;
-      size_t lds = 0;
-      for (int32_t ti : wl.tids) {
-        const DevTensor& d = plan.dev[ti];
-        lds = std::max(lds, small_lds(nt, d.N, d.factored ? d.R + d.C : 0));
+  if (plan.small[exact_norm]) {
+    for (const bool large : {false, true}) {
+      for (auto& kv : large ? plan.smallL : plan.smallS) {
+        const WorkList& wl = kv.second;
+        SmallFn fn;
+        if (large) CAME8_TYPE_SWITCH2(k_small_step_L, kv.first.pdt, kv.first.gdt, fn);
+        else CAME8_TYPE_SWITCH2(k_small_step_S, kv.first.pdt, kv.first.gdt, fn);
+        const int nt = large ? kLargeThreads : kSmallThreads;
+        size_t lds = 0;
+        for (int32_t ti : wl.tids) {
+          const DevTensor& d = plan.dev[ti];
+          lds = std::max(lds, small_lds(nt, d.N, d.factored ? d.R + d.C : 0));
+        }
+        PhaseTimer pt(PH_SMALL, alg_bytes(plan, wl, tensors, PH_SMALL), stream);
+        hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), dim3(nt), lds, stream, dT, tids(wl), int(wl.tids.size()),
+                           int(exact_norm), hp);
+        if ((rc = check_launch("small_step")) != CAME8_OK) return rc;
       }
-      PhaseTimer pt(PH_SMALL, alg_bytes(plan, wl, tensors, PH_SMALL), stream);
-      hipLaunchKernelGGL(fn, dim3(grid_for(wl.total())), dim3(nt), lds, stream, dT, tids(wl), int(wl.tids.size()),
-                         int(exact_norm), hp);
-      if ((rc = check_launch("small_step")) != CAME8_OK) return rc;
     }
+    return CAME8_OK;
   }
 
   // ---- P1 and 1-D pass A ----
@@ -1721,7 +1779,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     }
     if ((rc = launch_walk(plan.nwalk, plan.nfinal, stream)) != CAME8_OK) return rc;
   }
-  if ((exact_norm && (any_fact || !plan.vecA.empty())) || any2d) {  // reference order: only the 8bit2d tensors take this divisor
+  if (exact_norm || any2d) {  // reference order: only the 8bit2d tensors take this divisor
     PhaseTimer pt(PH_CLIP, 0.0, stream);
     hipLaunchKernelGGL(k_clip<>, dim3(grid_for(n_tensors)), blk, 0, stream, dT, int(n_tensors), int(!exact_norm), hp);
     if ((rc = check_launch("clip")) != CAME8_OK) return rc;
@@ -1845,7 +1903,7 @@ int came8_step_static(const came8_tensor* tensors, int32_t n_tensors, const came
   int rc = static_scratch(&ws);
   if (rc != CAME8_OK) return rc;
   size_t need = 0;
-  if ((rc = came8_workspace_size(tensors, n_tensors, hp->block_size, &need)) != CAME8_OK) return rc;
+  if ((rc = plan_size(tensors, n_tensors, hp->block_size, kStaticScratchBytes, &need)) != CAME8_OK) return rc;
   if (need > kStaticScratchBytes)
     return fail(CAME8_ESPACE, "came8_step_static: these tensors need " + std::to_string(need) +
                                   " bytes of scratch; the static scratch holds " + std::to_string(kStaticScratchBytes) +

@@ -1778,8 +1778,7 @@ __global__ __launch_bounds__(kThreads) void k_clip(const DevTensor* __restrict__
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   for (int k = blockIdx.x; k < ntens; k += gridDim.x) {
     const DevTensor& t = T[k];
-    // (uniform over the workgroup; a tensor without partials wrote its divisor itself, k_small_step)
-    if ((only2d && !t.mode2d) || t.nclip == 0) continue;
+    if (only2d && !t.mode2d) continue;  // uniform over the workgroup
     double s = 0.0;
     for (int64_t i = tid; i < t.nclip; i += kThreads) s += t.clip_part[i];
     s = wave_sum(s);

@@ -9,6 +9,7 @@ from came_amd import _lib
 from oracle import came8_oracle as orc
 from tests import parity as P
 from tests.test_gpu_parity import _tight_step_check
+from tests.test_gpu_side_stream import _static_step
 
 pytestmark = pytest.mark.gpu
 
@@ -58,11 +59,15 @@ def test_small_tensors(dtype, block, exact_norm):
 SHORT = [(1,), (2,), (3,), (4,), (5,), (6,), (7,), (8,), (12,), (13,), (14,), (15,), (127,), (129,), (2041,), (2042,),
          (2043,), (2044,), (2045,), (2046,), (2047,), (2048,), (1, 1), (1, 300), (300, 1), (5, 8), (64, 32), (45, 45),
          (2, 1024), (1024, 2), (1, 2048), (2048, 1), (1, 4, 500)]
-LONG = [(2049,), (4095,), (4096,), (4099,), (32761,), (32766,), (32767,), (32768,), (96, 200), (16, 1280), (1280, 16),
+LONG = [(2049,), (4095,), (4096,), (4099,), (20003,), (32761,), (32766,), (32767,), (32768,), (96, 200), (16, 1280), (1280, 16),
         (2547, 12), (12, 2548), (13, 2520), (64, 64), (65, 63), (181, 181), (256, 128), (127, 258), (31, 1057),
         (1, 2559), (2559, 1), (1, 40, 800), (1, 1, 16, 2032)]
 # just past an edge, each of which takes a whole call through the passes
 PAST = [(32769,), (129, 255), (13, 2548), (1, 2560), (2560, 1), (3, 40, 60)]
+
+
+def _count(shape):
+    return torch.Size(shape).numel()
 
 
 def _phases(step):
@@ -82,7 +87,7 @@ def _optimizer(cls, shapes, dtype=torch.float32, gdtype=None, offset=0, seed=5, 
     gen = torch.Generator().manual_seed(seed)
     ps = []
     for s in shapes:
-        n = torch.Size(s).numel()
+        n = _count(s)
         p = torch.empty(n + offset, device="cuda", dtype=dtype)[offset:].view(s)
         g = torch.empty(n + offset, device="cuda", dtype=gdtype or dtype)[offset:].view(s)
         p.copy_(torch.randn(s, generator=gen) * 0.02)
@@ -108,11 +113,63 @@ def test_calls_of_small_tensors_take_one_launch(shapes, cls):
         assert "small_step" not in ran and ran, s
 
 
+# (tensors, class, whether one launch takes them with the default clip, and with the exact one): both sides of each line
+# that the host draws where the passes are the faster (small_call)
+LINES = [([(4096,)], "CAME8bit", True, True), ([(4097,)], "CAME8bit", True, False),
+         ([(4097,)] * 191, "CAME8bit", True, False), ([(4097,)] * 192, "CAME8bit", True, True),
+         ([(8192,)], "CAMECUDA", True, True), ([(8193,)] * 63, "CAMECUDA", True, False),
+         ([(8193,)] * 64, "CAMECUDA", True, True), ([(128, 128), (16384,)], "CAME8bit", True, True),
+         ([(16, 1025)] * 95 + [(8,)] * 9, "CAME8bit", True, False), ([(16, 1025)] * 96, "CAME8bit", True, True),
+         ([(16, 1025)] * 63, "CAMECUDA", True, False), ([(16, 1025)] * 64, "CAMECUDA", True, True),
+         ([(28672,)], "CAME8bit", True, False), ([(28673,)] * 31, "CAME8bit", False, False),
+         ([(28673,)] * 32, "CAME8bit", True, False), ([(28673,)], "CAMECUDA", True, False),
+         ([(28673,), (8, 8)], "CAME8bit", True, False), ([(16, 1024)] * 640, "CAME8bit", True, True),
+         ([(16, 1024)] * 641, "CAME8bit", True, False), ([(16, 1023)] * 641, "CAME8bit", True, True),
+         ([(16, 2048)] * 768, "CAME8bit", True, False), ([(16, 2048)] * 769, "CAME8bit", False, False),
+         ([(16, 2048)] * 769, "CAMECUDA", True, True)]
+
+
+@pytest.mark.parametrize("line", LINES, ids=lambda c: f"{len(c[0])}x{c[0][0]}-{c[1]}")
+def test_lines_between_one_launch_and_the_passes(line):
+    """Each mode by itself and after the other one (the plan of a step serves both)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    shapes, cls, default, exact = line
+    _, opt = _optimizer(cls, shapes)
+    for mode, small in ((True, exact), (False, default), (True, exact)):
+        opt.exact_norm = mode
+        ran = _phases(opt.step)
+        assert ("small_step" in ran) == small and (ran == {"small_step"}) == small, (mode, ran)
+
+
+@pytest.mark.parametrize("shapes", [[(8192,), (16384,), (4099,)], [(96, 200), (181, 181), (9,)]], ids=["vectors", "matrices"])
+def test_modes_of_different_routes_match_the_oracle(shapes):
+    """The default clip in one launch, the exact one through the passes, of one set."""
+    for exact_norm in (False, True):
+        _run(came_amd.CAME8bitFull, shapes, torch.float32, 256, exact_norm, heavy=False, seed=17)
+
+
+def test_one_launch_where_the_passes_do_not_fit():
+    """A call that the passes would take, in a workspace that is too small for their scratch (the 32 MiB of the static
+    entry point): one launch, and the same step."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    shapes = [(16, 2048)] * 900
+    out = []
+    for entry in (lambda opt, ps: opt.step(), _static_step):
+        ps, opt = _optimizer("CAME8bit", shapes)
+        out.append((ps, opt, _phases(lambda: entry(opt, ps))))
+    assert "small_step" not in out[0][2] and out[1][2] == {"small_step"}
+    _same_steps([(ps, [opt.state[p] for p in ps]) for ps, opt, _ in out], shapes)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("block", [64, 100, 256, 4096])
 @pytest.mark.parametrize("exact_norm", [False, True])
 @pytest.mark.parametrize("shapes", [SHORT, LONG], ids=["short", "long"])
 def test_one_workgroup_steps(shapes, dtype, block, exact_norm):
+    if exact_norm:  # past 16384 elements it takes a crowd (test_one_launch_matches_the_passes)
+        shapes = [s for s in shapes if _count(s) <= 16384]
     heavy = block == 64 and dtype != torch.float16
     _run(came_amd.CAME8bitFull, shapes, dtype, block, exact_norm, heavy=heavy, seed=91)
 
@@ -124,7 +181,7 @@ def test_small_vectors_with_the_fp16_rounded_update(dtype, block):
     large tensor."""
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
-    shapes = [s for s in SHORT + LONG if len(s) == 1]
+    shapes = [s for s in SHORT + LONG if len(s) == 1 and s[0] <= 28672]
     params = P.make_params(shapes, dtype, seed=block)
     gen = torch.Generator().manual_seed(block + 1)
     hp = dict(HP, block_size=block)
@@ -170,7 +227,7 @@ def test_one_launch_matches_the_passes(route):
     route = dict(route)
     exact = route.pop("exact_norm", False)
     cls = route.pop("cls")
-    shapes = SHORT + LONG
+    shapes = SHORT + LONG + ([(181, 181), (31, 1057), (2547, 12), (20003,)] * 24 if exact else [])
     out = []
     for more in ([], [(300, 200)]):
         ps, opt = _optimizer(cls, shapes + more, **route)
