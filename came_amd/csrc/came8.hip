@@ -49,7 +49,14 @@ constexpr int kMaxShrink = 6;
 // No matrix is shrunk past this many bands: few workgroups add its partials per column (eight for 2048 columns), and
 // at 2000 bands of 32000x2048 that took 72 us twice a step.
 constexpr int64_t kMaxShrunkBands = 512;
-constexpr int64_t kFactorFewBlocks = 512;  // a factor launch of at most this many blocks takes eight wavefronts a block
+// A factor launch spreads its band sums over wavefronts (k_factor_blocks) where its tensors' most bands are at least
+// kSpreadBands and it has few blocks for them.  Both launches of a step, a thread a column and spread, us: 2048x2048 (256
+// bands, 16 blocks) 15.0 + 14.7 and 11.7 + 11.8; 32000x2048 (508, 133) 24.1 + 24.4 and 17.5 + 17.2; 24 of 1000x1000 (125, 192)
+// 13.9 + 13.6 and 12.2 + 12.4; a 1B-style model's layers (508, 749) 27.1 + 27.1 and 27.5 + 22.5; the other way 16 of 4096x4096
+// (128, 512) 13.6 + 13.8 and 18.2 + 14.5; 64 of 640x640 (40, 384) 10.4 + 10.5 and 15.0 + 11.5; 292 tensors of a 24-layer model
+// (393, 1745) 24.9 + 24.7 and 43.7 + 29.1.
+constexpr int64_t kSpreadBands = 96;
+bool factor_spread(int64_t bands, int64_t blocks) { return bands >= kSpreadBands && blocks * 5 <= bands * 8; }
 constexpr int64_t kMinLaunchBands = 2048;  // without a device to ask: the least work items per launch
 // Fixed time of a band (its start, its row sums, its partial stores), about 5 us, in elements the
 // whole GPU streams meanwhile: a workgroup among `slots` spends it as kBandFixedElems / slots.
@@ -1616,12 +1623,12 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     }
     return CAME8_OK;
   };
-  // Factor kernels: eight wavefronts share a block's band sums while the launch has few blocks, else four (a lone
-  // 2048x2048 in 256 bands: 14.5 + 12.9 -> 10.9 + 10.8 us; 1745 blocks of 292 tensors: four 22.6, eight 36.7 us)
-  auto launch_factor = [&](auto kernel4, auto kernel8, const WorkList& wl, size_t lds4, size_t lds8) {
-    const bool few = wl.total() <= kFactorFewBlocks;
-    hipLaunchKernelGGL(few ? kernel8 : kernel4, dim3(grid_for(wl.total())), dim3((few ? 8 : 4) * kWave),
-                       few ? lds8 : lds4, stream, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
+  auto launch_factor = [&](auto kernel, auto spread, const WorkList& wl, size_t lds) {
+    int64_t bands = 0;
+    for (int32_t ti : wl.tids) bands = std::max(bands, plan.dev[ti].nbands);
+    const bool sp = factor_spread(bands, wl.total());
+    hipLaunchKernelGGL(sp ? spread : kernel, dim3(grid_for(wl.total())), dim3((sp ? kSpreadWaves : 4) * kWave), sp ? lds : 0,
+                       stream, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
   };
   bool split = false;  // the long-chain group runs on the side stream (set by the clip-norm section)
 
@@ -1696,8 +1703,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
   if (any_factor) {
     const WorkList& fb = plan.factor;
     { PhaseTimer pt(PH_FACTOR, alg_bytes(plan, fb, tensors, PH_FACTOR), stream);
-    launch_factor(k_factor_blocks<false, 4>, k_factor_blocks<false, 8>, fb, factor_lds(4, exact_norm || any2d),
-                  factor_lds(8, exact_norm || any2d));
+    launch_factor(k_factor_blocks<false, false>, k_factor_blocks<false, true>, fb, factor_lds(exact_norm || any2d));
     if ((rc = check_launch("factor_blocks")) != CAME8_OK) return rc; }
   }
   if ((rc = launch_state_quant(k_state_quant<false>, "state_quant")) != CAME8_OK) return rc;
@@ -1819,7 +1825,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     if (any_factor) {
       const WorkList& fb = plan.factor;
       PhaseTimer pt(PH_FACTOR_RES, alg_bytes(plan, fb, tensors, PH_FACTOR_RES), stream);
-      launch_factor(k_factor_blocks<true, 4>, k_factor_blocks<true, 8>, fb, factor_lds(4, false), factor_lds(8, false));
+      launch_factor(k_factor_blocks<true, false>, k_factor_blocks<true, true>, fb, factor_lds(false));
       if ((rc = check_launch("factor_blocks_res")) != CAME8_OK) return rc;
     }
     if ((rc = launch_state_quant(k_state_quant<true>, "state_quant_res")) != CAME8_OK) return rc;

@@ -1174,15 +1174,16 @@ __device__ __forceinline__ float matrix_row_mean(const DevTensor& t, const float
   return row_mean_of_sum(t, ordered_sum_f64(bandsum + b * nb, nb, 1));
 }
 
-// A column block's sums over its band partials are spread over the workgroup's NW wavefronts: wavefront w adds
-// bands w, w + NW, ... of 256 columns (four a lane, every load 256 contiguous bytes, a batch of bands in flight), and
-// the wavefronts' fp64 sums are added in order through LDS.  One thread per column waited for nbands / 16 memory
-// round trips.  NW is 4 (every thread finishes a column), or 8 where a launch has too few blocks to occupy the GPU
-// with those (came8.hip; 16 spill).
+// A column block's sums over its band partials take one of two forms.  A thread a column, sixteen bands in flight: it
+// waits for nbands / 16 memory round trips, which other workgroups cover where a launch has many blocks.  Spread: over
+// kSpreadWaves wavefronts, wavefront w adding bands w, w + kSpreadWaves, ... of 256 columns (four a lane, every load 256
+// contiguous bytes, a batch of bands in flight), whose fp64 sums are added in order through LDS.  The host takes the
+// second for many bands in few blocks (factor_spread in came8.hip).
 constexpr int kFactorCols = 256;
-// LDS of a launch: the wavefronts' sums of one or two partial arrays
-constexpr size_t factor_lds(int nw, bool two_arrays) {
-  return sizeof(double) * nw * kFactorCols * (two_arrays ? 2 : 1);
+constexpr int kSpreadWaves = 8;  // (16 spill)
+// LDS of a spread launch: the wavefronts' sums of one or two partial arrays
+constexpr size_t factor_lds(bool two_arrays) {
+  return sizeof(double) * kSpreadWaves * kFactorCols * (two_arrays ? 2 : 1);
 }
 
 // row of row state / column of column state i of a tensor, and its matrix
@@ -1243,11 +1244,42 @@ __device__ __forceinline__ void band_column_part(const DevTensor& t, const float
     for (int q = 0; q < 4; ++q) psum[(x * NW + wid) * kFactorCols + q * kWave + lane] = acc[x][q];
 }
 
-template <bool RES, int NW>
-__global__ __launch_bounds__(NW * kWave) void k_factor_blocks(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
-                                                                  const int64_t* __restrict__ wstart, int ntens, Hp hp) {
-  constexpr int NA = RES ? 1 : 2;
-  extern __shared__ double psum[];  // [array][wavefront][column] (factor_lds)
+// U bands from k on of a column's partials (stride C), by one thread (LAST: past the last band that one again, not
+// counted)
+template <int NA, int U, bool LAST>
+__device__ __forceinline__ void column_bands(const CAME8_GLOBAL float* g0, const CAME8_GLOBAL float* g1, int k, int n,
+                                             int64_t C, double (&acc)[NA]) {
+  float v[NA][U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int64_t o = int64_t(LAST ? min(k + u, n - 1) : k + u) * C;
+    v[0][u] = g0[o];
+    if constexpr (NA > 1) v[NA - 1][u] = g1[o];
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int x = 0; x < NA; ++x) acc[x] += !LAST || k + u < n ? double(v[x][u]) : 0.0;
+}
+// The sums over a column's n bands of one or two arrays, by one thread in band order.  The last ones go four at a time:
+// most of sixteen loads would be in vain for a matrix of two bands (512 of 16x2048: 33.6 us in eights, 23 in fours).
+template <int NA>
+__device__ __forceinline__ void column_sums(const float* __restrict__ p0, const float* __restrict__ p1, int n, int64_t C,
+                                            double (&acc)[NA]) {
+  const CAME8_GLOBAL float* __restrict__ g0 = gbl(p0);
+  const CAME8_GLOBAL float* __restrict__ g1 = NA > 1 ? gbl(p1) : g0;
+  int k = 0;
+#pragma unroll 1
+  for (; k + kSumBatch <= n; k += kSumBatch) column_bands<NA, kSumBatch, false>(g0, g1, k, n, C, acc);
+#pragma unroll 1
+  for (; k < n; k += 4) column_bands<NA, 4, true>(g0, g1, k, n, C, acc);
+}
+
+template <bool RES, bool SPREAD>
+__global__ __launch_bounds__((SPREAD ? kSpreadWaves : 4) * kWave) void k_factor_blocks(
+    const DevTensor* __restrict__ T, const int32_t* __restrict__ tids, const int64_t* __restrict__ wstart, int ntens, Hp hp) {
+  constexpr int NA = RES ? 1 : 2, NW = SPREAD ? kSpreadWaves : 4;
+  extern __shared__ double psum[];  // SPREAD: [array][wavefront][column] (factor_lds)
   __shared__ float smax[NW];
   __shared__ double ssum[NW], msum[NW];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -1350,10 +1382,19 @@ __global__ __launch_bounds__(NW * kWave) void k_factor_blocks(const DevTensor* _
         if (RES && t.mode2d) {
           // 8bit2d: a float32 sum from zero over the tile rows in order (the reference's), 16 loads at a time
           if (own) s = ordered_sum_f32(t.t2col + i, t.tr, t.C);
-        } else if (t.nbands == 1) {  // one band a matrix (small matrices): its partial is the sum
+        } else if constexpr (!SPREAD) {
           if (own) {
-            s = part[i];
-            if (withW) W = double(t.partW[i]);
+            const int64_t b = col_matrix(t, i), o = (b * t.nbands) * t.C + (i - b * t.C);
+            if (withW) {
+              double sw[NA] = {};
+              column_sums<NA>(part + o, t.partW + o, int(t.nbands), t.C, sw);
+              s = float(sw[0]);
+              W = sw[NA - 1];
+            } else {
+              double sw[1] = {};
+              column_sums<1>(part + o, nullptr, int(t.nbands), t.C, sw);
+              s = float(sw[0]);
+            }
           }
         } else {
           const bool one = col_matrix(t, min(cb + kFactorCols, i1) - 1) == col_matrix(t, cb);  // uniform
@@ -1393,7 +1434,7 @@ __global__ __launch_bounds__(NW * kWave) void k_factor_blocks(const DevTensor* _
             csum += double(crm) * double(c) * double(c) * W;
           }
         }
-        if (cb + kFactorCols < i1) __syncthreads();  // psum is written again
+        if (SPREAD && cb + kFactorCols < i1) __syncthreads();  // psum is written again
       }
     }
     // block max and clip partial (fixed order)

@@ -38,6 +38,20 @@ def test_tiny_matrices(dtype, block, exact_norm):
     _run(came_amd.CAME8bitFull, TINY, dtype, block, exact_norm, heavy=block == 256, seed=71)
 
 
+# Many row bands in few state blocks, whose column sums are spread over wavefronts, and the same matrix among others, whose
+# columns a thread adds: band counts with every remainder of its batches of sixteen and four, blocks over several matrices
+BANDS = [(1000, 300)]
+COLUMNS = [(1000, 300)] * 12 + [(8 * k + r, 264) for k, r in ((1, 0), (1, 1), (3, 7), (4, 0), (15, 8), (16, 1), (18, 8), (35, 0))] + [
+    (5, 200, 40), (70, 24, 9), (3, 130, 300)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("exact_norm", [False, True])
+@pytest.mark.parametrize("shapes", [BANDS, COLUMNS], ids=["spread", "columns"])
+def test_band_sums(shapes, dtype, exact_norm):
+    _run(came_amd.CAME8bitFull, shapes, dtype, 64, exact_norm, heavy=False, seed=33)
+
+
 # Small and just larger tensors in one call: the larger ones take them all through the passes, with rows of fewer and more
 # columns than threads and lengths with every tail of the norm's chains.
 SMALL = [(1,), (7,), (12,), (4095,), (4096,), (4099,), (32768,), (32769,), (1, 1), (1, 300), (300, 1), (5, 8), (96, 200),
