@@ -117,7 +117,7 @@ struct Plan {
   std::map<BandKey, WorkList> band2;     // P2 (factored tensors of the full8bit / fp32 layouts)
   std::map<int, WorkList> tiny1;         // P1 of tensors of tiny matrices (per ngrp matrices), by grad type
   std::map<int, WorkList> tiny2;         // P2 of tensors of tiny matrices, by grad type
-  WorkList tinyq;                        // their states' codes (per four state blocks)
+  WorkList tinyq;                        // their states' codes (per four state blocks, or per long one)
   // small tensors, a workgroup each for the whole step, by types: up to kSmallElems elements, and larger ones
   std::map<TypeKey, WorkList> smallS, smallL;
   bool small[2] = {false, false};        // [exact clip]: those lists are the step, not the passes (small_call)
@@ -736,7 +736,7 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, size
       if (tiny_matrix(t, false)) {
         add_item(plan.tiny1[t.grad_dtype], i, d.nclip);
         add_item((longc[i] ? plan.tiny2L : plan.tiny2)[t.grad_dtype], i, d.nclip);
-        if (!d.fp32st) add_item(plan.tinyq, i, ceil_div(d.nbr + d.nbc, int64_t(4)));
+        if (!d.fp32st) add_item(plan.tinyq, i, B > kStateWaveMax ? d.nbr + d.nbc : ceil_div(d.nbr + d.nbc, int64_t(4)));
       } else {
         const bool pm_m = d.pm && (d.R * d.C) % B != 0;
         const BandShapeSel sel1 = band_variant(t, d.C, B, 1), sel2 = band_variant(t, d.C, B, 2, pm_m);
@@ -1586,10 +1586,10 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     for (int32_t ti : wl.tids) bytes = std::max(bytes, tiny_lds(plan.dev[ti].R * plan.dev[ti].C, codes));
     return bytes;
   };
-  auto launch_state_quant = [&](auto kernel, const char* what) -> int {
+  auto launch_state_quant = [&](auto kernel, auto wide, const char* what) -> int {
     if (plan.tinyq.tids.empty()) return CAME8_OK;
     const WorkList& wl = plan.tinyq;
-    hipLaunchKernelGGL(kernel, dim3(grid_for(wl.total())), blk, 0, stream, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
+    hipLaunchKernelGGL(h.block_size > kStateWaveMax ? wide : kernel, dim3(grid_for(wl.total())), blk, 0, stream, dT, tids(wl), wst(wl), int(wl.tids.size()), hp);
     return check_launch(what);
   };
   // P2 of one group of factored tensors: through the pass's queues, or all on queue q
@@ -1706,7 +1706,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
     launch_factor(k_factor_blocks<false, false>, k_factor_blocks<false, true>, fb, factor_lds(exact_norm || any2d));
     if ((rc = check_launch("factor_blocks")) != CAME8_OK) return rc; }
   }
-  if ((rc = launch_state_quant(k_state_quant<false>, "state_quant")) != CAME8_OK) return rc;
+  if ((rc = launch_state_quant(k_state_quant<false, false>, k_state_quant<false, true>, "state_quant")) != CAME8_OK) return rc;
   // ---- clip divisor ----
   if (!exact_norm) {  // the update norm in the reference's order (came8_norm.h)
     using EstFn = void (*)(const DevTensor*, const int32_t*, const int64_t*, int, Hp);
@@ -1828,7 +1828,7 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
       launch_factor(k_factor_blocks<true, false>, k_factor_blocks<true, true>, fb, factor_lds(false));
       if ((rc = check_launch("factor_blocks_res")) != CAME8_OK) return rc;
     }
-    if ((rc = launch_state_quant(k_state_quant<true>, "state_quant_res")) != CAME8_OK) return rc;
+    if ((rc = launch_state_quant(k_state_quant<true, false>, k_state_quant<true, true>, "state_quant_res")) != CAME8_OK) return rc;
   }
   // ---- P3 and 1-D pass B ----
   for (auto& kv : plan.param2d_v) {

@@ -1688,18 +1688,22 @@ __global__ __launch_bounds__(kThreads) void k_tiny_pass2(const DevTensor* __rest
   }
 }
 
-// Codes of the row and column states that the tiny passes formed (RES: the residual ones): a wavefront per
-// state block, four blocks a work item.
-template <bool RES>
+// Codes of the row and column states that the tiny passes formed (RES: the residual ones): a wavefront per state block,
+// four blocks a work item, or (WIDE: blocks of more than kStateWaveMax) a workgroup, since tensors of few long blocks
+// wait for a wavefront's loads of its block one after the other.
+constexpr int kStateWaveMax = 512;
+template <bool RES, bool WIDE>
 __global__ __launch_bounds__(kThreads) void k_state_quant(const DevTensor* __restrict__ T, const int32_t* __restrict__ tids,
                                                           const int64_t* __restrict__ wstart, int ntens, Hp hp) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  constexpr int kStep = WIDE ? kThreads : kWave;  // lanes of a block
+  __shared__ float wm[4];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, first = WIDE ? int(threadIdx.x) : lane;
   const int64_t total = wstart[ntens];
   for (int64_t w = blockIdx.x; w < total; w += gridDim.x) {
     const int slot = find_slot(wstart, ntens, w);
     const DevTensor& t = T[tids[slot]];
-    const int64_t local = (w - wstart[slot]) * 4 + wid;
-    if (local >= t.nbr + t.nbc) continue;  // uniform over the wavefront; no barrier below
+    const int64_t local = WIDE ? w - wstart[slot] : (w - wstart[slot]) * 4 + wid;
+    if (local >= t.nbr + t.nbc) continue;  // uniform over the wavefront, never taken where a barrier follows (WIDE)
     const bool is_row = local < t.nbr;
     const int64_t blk = is_row ? local : local - t.nbr;
     const int64_t n = is_row ? t.R : t.C, len = t.P * n;
@@ -1714,27 +1718,34 @@ __global__ __launch_bounds__(kThreads) void k_state_quant(const DevTensor* __res
     }
     const CAME8_GLOBAL float* __restrict__ src = gbl(static_cast<const float*>(is_row ? (RES ? t.RRn : t.Rn) : (RES ? t.CRn : t.Cn)));
     CAME8_GLOBAL uint8_t* __restrict__ q = gbl((is_row ? t.rq : t.cq) + (RES ? len : 0));
-    constexpr int kHeld = 4;  // states a lane holds (blocks of 256); later ones are read again
+    constexpr int kHeld = 4;  // states a lane holds; later ones are read again
     float v[kHeld];
     float vmax = (i1 - i0) < hp.B ? 0.0f : -__builtin_inff();  // zero padding joins the max
 #pragma unroll
     for (int k = 0; k < kHeld; ++k) {
-      const int64_t i = i0 + lane + k * kWave;
+      const int64_t i = i0 + first + k * kStep;
       v[k] = src[min(i, i1 - 1)];  // past the end: the last state again
       vmax = nan_max(vmax, v[k]);
     }
-    for (int64_t i = i0 + lane + kHeld * kWave; i < i1; i += kWave) vmax = nan_max(vmax, src[i]);
-    const float amax = fix_absmax(group_max<64>(vmax)), arcp = rcp_for_div(amax);
-    if (lane == 0) {
+    for (int64_t i = i0 + first + kHeld * kStep; i < i1; i += kStep) vmax = nan_max(vmax, src[i]);
+    vmax = group_max<64>(vmax);
+    if constexpr (WIDE) {
+      if (lane == 0) wm[wid] = vmax;
+      __syncthreads();
+      vmax = nan_max(nan_max(wm[0], wm[1]), nan_max(wm[2], wm[3]));
+      __syncthreads();  // wm is written again by the next item
+    }
+    const float amax = fix_absmax(vmax), arcp = rcp_for_div(amax);
+    if (first == 0) {
       if (is_row) t.ra[(RES ? t.nbr : 0) + blk] = amax;
       else t.ca[(RES ? t.nbc : 0) + blk] = amax;
     }
 #pragma unroll
     for (int k = 0; k < kHeld; ++k) {
-      const int64_t i = i0 + lane + k * kWave;
+      const int64_t i = i0 + first + k * kStep;
       if (i < i1) q[i] = quant_u8_r(v[k], amax, arcp);
     }
-    for (int64_t i = i0 + lane + kHeld * kWave; i < i1; i += kWave) q[i] = quant_u8_r(src[i], amax, arcp);
+    for (int64_t i = i0 + first + kHeld * kStep; i < i1; i += kStep) q[i] = quant_u8_r(src[i], amax, arcp);
   }
 }
 
