@@ -14,8 +14,7 @@ from tests.test_gpu_side_stream import _static_step
 pytestmark = pytest.mark.gpu
 
 HP = dict(lr=1e-3, weight_decay=1e-2)
-# matrices of 1 to 64 elements, around the counts staged at a time (256; 128 above 48 elements), and one item of
-# several batches' worth of matrices
+# matrices of 1 to 64 elements, around the counts staged at a time and of a work item (256; 128 above 48 elements)
 TINY = [(1, 1, 1), (255, 3, 3), (256, 3, 3), (257, 1, 1), (129, 7, 7), (128, 8, 8), (300, 2, 31), (513, 6, 8),
         (40, 30, 5, 5), (4099, 3, 1)]
 
@@ -36,6 +35,12 @@ def _run(cls, shapes, dtype, block, exact_norm, heavy, seed):
 @pytest.mark.parametrize("exact_norm", [False, True])
 def test_tiny_matrices(dtype, block, exact_norm):
     _run(came_amd.CAME8bitFull, TINY, dtype, block, exact_norm, heavy=block == 256, seed=71)
+
+
+@pytest.mark.parametrize("exact_norm", [False, True])
+def test_items_of_several_batches(exact_norm):
+    """Above 4096 work items of 256 matrices an item takes more of them."""
+    _run(came_amd.CAME8bitFull, [(256 * 4096 + 300, 1, 1), (9, 3, 3)], torch.bfloat16, 256, exact_norm, heavy=False, seed=72)
 
 
 # Many row bands in few state blocks, whose column sums are spread over wavefronts, and the same matrix among others, whose
