@@ -1991,16 +1991,20 @@ int came8_quantize_blockwise(const float* x, int64_t n, int32_t is_signed, int32
   if (!absmax || (n > 0 && (!x || !q))) return fail(CAME8_EINVAL, "came8_quantize_blockwise: null pointer");
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   const int64_t nb = std::max<int64_t>(1, ceil_div(n, block_size));
+  // k_quantize_p2 wherever its loads fit, but for few short blocks, whose latency counts (us: 11008x4096 in blocks of 256
+  // 43 and 77 in k_quantize_any, 2^20 elements 4.6 and 4.2, 2^18 4.5 and 3.5, one block 3.7 and 2.5; 128 blocks of 2048
+  // 4.3 and 4.8).  There a workgroup per block is the faster up to five blocks an element of one (256 blocks of 1000 3.8,
+  // 6.9 a wavefront each; 8192 of 256 8.7 and 5.2).
   const bool pow2 = (block_size & (block_size - 1)) == 0;
-  // k_quantize_p2 wherever its loads fit (44 us against 176 on 11008x4096 in blocks of 256)
-  if (pow2 && block_size >= 4 && block_size <= kQuantTile && n > 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+  const bool few = n <= kQuantFewElems && nb <= 8192 && block_size <= 1024;
+  if (!few && pow2 && block_size >= 4 && block_size <= kQuantTile && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(q) % 4 == 0) {
     hipLaunchKernelGGL(is_signed ? k_quantize_p2<true> : k_quantize_p2<false>, dim3(grid_for(ceil_div(n, kQuantTile))),
                        dim3(kThreads), 0, stream, x, n, log2_or_minus1(block_size), q, absmax);
   } else {
-    const int64_t items = block_size > kQuantWaveMax ? nb : ceil_div(nb, 4);
-    hipLaunchKernelGGL(is_signed ? k_quantize_any<true> : k_quantize_any<false>, dim3(grid_for(items)), dim3(kThreads),
-                       0, stream, x, n, block_size, nb, q, absmax);
+    const bool wide = block_size > 1024 || (block_size >= 128 && nb <= 5 * int64_t(block_size));
+    hipLaunchKernelGGL(is_signed ? k_quantize_any<true> : k_quantize_any<false>, dim3(grid_for(wide ? nb : ceil_div(nb, 4))),
+                       dim3(kThreads), 0, stream, x, n, block_size, nb, wide, q, absmax);
   }
   return check_launch("quantize");
 }
@@ -2013,9 +2017,9 @@ int came8_dequantize_blockwise(const void* q, const float* absmax, int64_t n, in
   if (!q || !absmax || !out) return fail(CAME8_EINVAL, "came8_dequantize_blockwise: null pointer");
   hipStream_t stream = static_cast<hipStream_t>(stream_ptr);
   const bool pow2 = (block_size & (block_size - 1)) == 0;
-  // k_dequantize_v4 wherever its loads fit (32 us against 76); the magic division of block sizes that are not
-  // powers of two takes indices below 2^31
-  if (block_size % 4 == 0 && (pow2 || n < (int64_t(1) << 31)) && reinterpret_cast<uintptr_t>(q) % 4 == 0 &&
+  // k_dequantize_v4 wherever its loads fit, but for the smallest calls (us: 11008x4096 32 and 76, 2^20 elements 3.2 and 3.7,
+  // 2^19 3.0 and 2.9, 2^16 2.8 and 2.5); the magic division of block sizes that are not powers of two takes indices below 2^31
+  if (n > kQuantFewElems && block_size % 4 == 0 && (pow2 || n < (int64_t(1) << 31)) && reinterpret_cast<uintptr_t>(q) % 4 == 0 &&
       reinterpret_cast<uintptr_t>(out) % 16 == 0) {
     uint64_t mB = 1;
     uint32_t sB = 0;

@@ -2967,6 +2967,7 @@ __device__ __forceinline__ uint32_t quant_code(float x, float a, float rcp, bool
 // rounds, or over wavefronts through LDS (B > 1024), and each element is read once.  11008x4096, B = 256: 44 us
 // (5.1 TB/s) against 176 us with a workgroup per block, an element a thread.
 constexpr int kQuantTile = 4096;
+constexpr int64_t kQuantFewElems = 1 << 19;  // up to these the launches of came8.hip count latency
 template <bool SIGNED>
 __global__ __launch_bounds__(kThreads) void k_quantize_p2(const float* __restrict__ x, int64_t n, int32_t log2B,
                                                           void* __restrict__ q, float* __restrict__ absmax) {
@@ -3041,16 +3042,14 @@ __global__ __launch_bounds__(kThreads) void k_quantize_p2(const float* __restric
   }
 }
 
-// Any block size and alignment: blocks of at most kQuantWaveMax elements take a wavefront each, longer ones a
-// workgroup; a block's elements are read again (from cache) once its maximum is known.
-constexpr int kQuantWaveMax = 1024;
+// Any block size and alignment: a wavefront per block, or (wide) a workgroup; a block's elements are read again (from
+// cache) once its maximum is known.
 template <bool SIGNED>
 __global__ __launch_bounds__(kThreads) void k_quantize_any(const float* __restrict__ x, int64_t n, int32_t B,
-                                                           int64_t nblocks, void* __restrict__ q,
+                                                           int64_t nblocks, bool wide, void* __restrict__ q,
                                                            float* __restrict__ absmax) {
   __shared__ float wm[4];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const bool wide = B > kQuantWaveMax;
   const int step = wide ? kThreads : kWave, first = wide ? tid : lane;
   const int64_t items = wide ? nblocks : (nblocks + 3) / 4;
   for (int64_t it = blockIdx.x; it < items; it += gridDim.x) {

@@ -54,3 +54,43 @@ def test_special_blocks(block, signed):
     rows[7] = -rows[7].abs()  # unsigned: a negative maximum
     rows[8, 3] = -1e30
     _check(rows.reshape(-1)[: 9 * block - 1], signed, block)
+
+
+@pytest.mark.parametrize("n", [2**19, 2**19 + 1, 2**19 + 3 * 4096 + 1021])
+@pytest.mark.parametrize("block", [4, 8, 64, 128, 256, 512, 1000, 1024, 1028, 2048, 4096, 8192])
+@pytest.mark.parametrize("signed", [True, False])
+def test_forms_of_many_elements_match_the_oracle(n, block, signed):
+    """Both sides of the size from which the vector tiles are taken, which the tests above stay below."""
+    test_forms_match_the_oracle(n, block, signed)
+
+
+@pytest.mark.parametrize("block", [4, 64, 256, 512, 1024, 2048, 4096])
+@pytest.mark.parametrize("signed", [True, False])
+def test_special_blocks_among_many(block, signed):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    gen = torch.Generator().manual_seed(block)
+    rows = torch.randn(2**19 // block + 7, block, generator=gen)
+    at = torch.randperm(rows.shape[0], generator=gen)[: 9 * 12].view(9, 12)
+    rows[at[0]] *= 1e-42
+    rows[at[1]] *= 1e-30
+    rows[at[2]] *= 1e25
+    rows[at[3], 2] = float("inf")
+    rows[at[4], 3] = float("nan")
+    rows[at[5], 1], rows[at[5], 2], rows[at[5], 3] = float("inf"), float("nan"), -float("inf")
+    rows[at[6]] = 0.0
+    rows[at[7]] = -rows[at[7]].abs()
+    rows[at[8], 3] = -1e30
+    _check(rows.reshape(-1)[: rows.numel() - 1], signed, block)
+
+
+@pytest.mark.parametrize("block,few", [(128, 640), (256, 1280), (1000, 5000), (1024, 5120), (64, 8192), (100, 8192)])
+def test_workgroup_and_wavefront_blocks(block, few):
+    """Around the block counts up to which a block of the general form takes a workgroup."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    for nb in (few, few + 1):
+        gen = torch.Generator().manual_seed(nb)
+        x = torch.randn(nb * block - 3, generator=gen)
+        _check(x, True, block, 1)
+        _check(x.abs(), False, block, 0)
