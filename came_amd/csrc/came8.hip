@@ -46,9 +46,12 @@ int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // estimate of the launch (band_shrinks).
 constexpr int64_t kMinShrunkBandRows = 8;
 constexpr int kMaxShrink = 6;
-// No matrix is shrunk past this many bands: few workgroups add its partials per column (eight for 2048 columns), and
-// at 2000 bands of 32000x2048 that took 72 us twice a step.
-constexpr int64_t kMaxShrunkBands = 512;
+// Bands a matrix has at most (more above 131072 rows, where bands have kMaxBandRows): each writes its column partials, which
+// few workgroups add (eight for 2048 columns).  It binds shrunk bands, and those that a wide matrix would have without: a step
+// over 20000x131072 with the exact clip takes 7.6 ms in 500 bands of 40 rows and 9.6 in 2500 of 8, 5000x262144 4.6 and 6.2.
+// 512, 1024 and unlimited, us a step:
+// one 32000x2048 403, 385, 384 (fp32 508, 534, 575), four of them 872, 952, 953, 50257x1024 384, 370, 445, 200000x512 777, 716, 960.
+constexpr int64_t kMaxMatrixBands = 512;
 // A factor launch spreads its band sums over wavefronts (k_factor_blocks) where its tensors' most bands are at least
 // kSpreadBands and it has few blocks for them.  Both launches of a step, a thread a column and spread, us: 2048x2048 (256
 // bands, 16 blocks) 15.0 + 14.7 and 11.7 + 11.8; 32000x2048 (508, 133) 24.1 + 24.4 and 17.5 + 17.2; 24 of 1000x1000 (125, 192)
@@ -64,13 +67,13 @@ constexpr int64_t kMinLaunchBands = 2048;  // without a device to ask: the least
 constexpr double kBandFixedElems = 8.4e6;
 
 // Rows per band: about 1M elements per workgroup work item, whole rows, at most 256 rows, divided by
-// 2^shrink.  Every band writes one fp32 partial per column and statistic, which the factor kernels
-// read back, so the band size sets that traffic (8-12 bytes per column per band).
+// 2^shrink, and at least as many as keep kMaxMatrixBands.  Every band writes one fp32 partial per column and statistic, which
+// the factor kernels read back, so the band size sets that traffic (8-12 bytes per column per band).
 int64_t band_rows(int64_t R, int64_t C, int shrink = 0) {
   int64_t rb = std::max<int64_t>(1, (int64_t(1) << 20) / std::max<int64_t>(C, 1));
   rb = std::min<int64_t>(rb, kMaxBandRows);
   rb = std::max<int64_t>(std::min<int64_t>(rb, kMinShrunkBandRows), rb >> shrink);
-  rb = std::max<int64_t>(rb, std::min<int64_t>(kMaxBandRows, ceil_div(R, kMaxShrunkBands)));
+  rb = std::max<int64_t>(rb, std::min<int64_t>(kMaxBandRows, ceil_div(R, kMaxMatrixBands)));
   return std::min<int64_t>(rb, R);
 }
 
