@@ -3,18 +3,20 @@
  * accumulation order of torch's CPU norm(2) (came_amd/csrc/came8_norm.h), written to check its
  * exactness argument against the serial chain on adversarial inputs.  Test infrastructure only.
  *
- * Segment records follow the kernel's rules: a segment holds 512 chain elements; lane l (64 lanes)
- * accounts elements 64q + l (q < 8) in an fp32 running sum of rint(x*x * 2^(23-E)) and the largest
- * |dh - rint(dh)|; a lane's value saturates at 2^24 for a tie (0.5), a sum of 2^24 or more (or NaN), or
- * a nonzero sum in the subnormal binade; the segment's value is the lanes' integer sum, at most 2^24.
- * In the subnormal binade (E = -126, unit 2^-149) an element |x| = 2^-75 also counts as a tie: its
- * square 2^-150 is half a unit, which x*x rounds to 0.
+ * Segment records follow the kernel's rules: a segment holds 512 chain elements; lane l of `lanes` (64, or
+ * the 16 of the kernel that takes several segments a wavefront) accounts elements lanes * q + l in two fp32
+ * sums of fused multiply-adds, one started at 2^E (even mantissa) and one a unit 2^(E-23) above it (odd).  A
+ * lane's value is the first sum less its start in units, or 2^24 when that is 2^23 or more (the sum left the
+ * binade, or met a NaN or an infinity), when the sums are not one unit apart any more (a tie, which rounds to
+ * the even side), or for E = 128, the binade above the largest; the segment's value is the lanes' integer
+ * sum, at most 2^24.
  * The walk skips a segment whose record covers the chain's binade when m + value < 2^24 and replays
  * the others.  A replay (segment_replay) follows the kernel's wavefront form: lane l holds the chain
- * elements 8l .. 8l + 7 of the segment; each round takes every element's integer increment under the
- * chain's current binade, a saturating prefix over lanes and elements, and the first element where the
- * prefix leaves the binade or the element is special; the elements before it are one integer add, that
- * element is one fmaf, and the next round starts after it.
+ * elements 8l .. 8l + 7 of the segment; each round takes every lane's increments under the chain's current
+ * binade as prefixes from the same pair of sums (elements already applied count as 0), a saturating prefix of
+ * the lanes' totals, and the first element where a lane's pair shows an exception or the prefix leaves the
+ * binade; the elements before it are one integer add, that element is one fmaf, and the next round starts
+ * after it.  A chain at zero takes its elements one by one.
  */
 #include <math.h>
 #include <stdint.h>
@@ -32,23 +34,33 @@ static int est_binade(double v) {
   if (!(v <= 0x1.fffffep127)) return 127;
   return binade((float)v);
 }
-static uint32_t seg_value(const float* x, int64_t k0, int64_t cnt, int E) {
+static float from_bits(uint32_t b) {
+  float v;
+  memcpy(&v, &b, 4);
+  return v;
+}
+static uint32_t to_bits(float v) {
+  uint32_t b;
+  memcpy(&b, &v, 4);
+  return b;
+}
+static uint32_t lane_value(float even, float odd, int E) {
+  const uint32_t base = (uint32_t)(E + 127) << 23;
+  const uint32_t n = to_bits(even) - base;
+  return n < (1u << 23) && to_bits(odd) - base == n + 1u && E < 128 ? n : (1u << 24);
+}
+/* the record of cnt <= 512 chain elements x[0 .. cnt) under binade E (-126 .. 128) */
+uint32_t seg_value(const float* x, int64_t cnt, int E, int lanes) {
+  const uint32_t base = (uint32_t)(E + 127) << 23;
   uint64_t tot = 0;
-  for (int lane = 0; lane < 64; ++lane) {
-    float sum = 0.0f, rmax = 0.0f;
-    for (int q = 0; q < 8; ++q) {
-      int64_t k = 64 * q + lane;
-      if (k >= cnt) continue;
-      float v = x[k0 + k];
-      float hi = v * v;
-      float dh = ldexpf(hi, 23 - E);
-      float nf = rintf(dh);
-      sum += nf;
-      rmax = fmaxf(rmax, fabsf(dh - nf));
-      if (E == -126 && fabsf(v) == 0x1p-75f) rmax = 0.5f; /* x*x = 2^-150 rounds to 0 but is a tie */
+  for (int lane = 0; lane < lanes; ++lane) {
+    float even = from_bits(base), odd = from_bits(base + 1u);
+    for (int64_t k = lane; k < 512; k += lanes) {
+      const float v = k < cnt ? x[k] : 0.0f;
+      even = fmaf(v, v, even);
+      odd = fmaf(v, v, odd);
     }
-    int bad = !(sum < 0x1p24f) || rmax == 0.5f || (E == -126 && sum != 0.0f);
-    tot += bad ? (1u << 24) : (uint32_t)sum;
+    tot += lane_value(even, odd, E);
   }
   return tot > (1u << 24) ? (1u << 24) : (uint32_t)tot;
 }
@@ -58,15 +70,14 @@ static uint32_t sat_add(uint32_t a, uint32_t b) {
   uint32_t v = a + b;
   return v < SAT ? v : SAT;
 }
-static float value_of(uint32_t m, int E) {
-  uint32_t r = ((uint32_t)(E + 126) << 23) + m;
-  float v;
-  memcpy(&v, &r, 4);
-  return v;
-}
+static float value_of(uint32_t m, int E) { return from_bits(((uint32_t)(E + 126) << 23) + m); }
 
 /* one segment of cnt <= 512 chain elements x[0 .. cnt) from s; *rounds counts the rounds */
 float segment_replay(const float* x, int cnt, float s, int64_t* rounds) {
+  if (s == 0.0f) {
+    for (int k = 0; k < cnt; ++k) s = fmaf(x[k], x[k], s);
+    return s;
+  }
   int pos = 0;
   while (pos < cnt) {
     ++*rounds;
@@ -79,39 +90,27 @@ float segment_replay(const float* x, int cnt, float s, int64_t* rounds) {
       break;
     }
     const int E = binade(s);
-    uint32_t b;
-    memcpy(&b, &s, 4);
-    const uint32_t m = b - ((uint32_t)(E + 126) << 23);
+    const uint32_t m = to_bits(s) - ((uint32_t)(E + 126) << 23);
     const uint32_t room = (1u << 24) - m;
-    uint32_t incl[512], run[64], excl[64];
-    int special[512];
+    const uint32_t base = (uint32_t)(E + 127) << 23;
+    uint32_t incl[512], excl[64], acc = 0;
+    int event[512];
     for (int lane = 0; lane < 64; ++lane) {
-      uint32_t r = 0;
+      float even = from_bits(base), odd = from_bits(base + 1u);
       for (int j = 0; j < 8; ++j) {
         const int k = lane * 8 + j;
-        const int live = k >= pos && k < cnt;
-        const float v = k < cnt ? x[k] : 0.0f;
-        const float h = v * v;
-        const float dh = ldexpf(h, 23 - E);
-        const float nf = rintf(dh);
-        uint32_t n = nf < 0x1p25f ? (uint32_t)nf : SAT;
-        special[k] = live && (fabsf(dh - nf) == 0.5f || (E == -126 && (nf != 0.0f || fabsf(v) == 0x1p-75f)));
-        r = sat_add(r, live ? n : 0u);
-        incl[k] = r;
+        const float v = k >= pos && k < cnt ? x[k] : 0.0f;
+        even = fmaf(v, v, even);
+        odd = fmaf(v, v, odd);
+        incl[k] = to_bits(even) - base;
+        event[k] = incl[k] >= (1u << 23) || to_bits(odd) - base != incl[k] + 1u;
       }
-      run[lane] = r;
-    }
-    uint32_t acc = 0;
-    for (int lane = 0; lane < 64; ++lane) {
       excl[lane] = acc;
-      acc = sat_add(acc, run[lane]);
+      acc = sat_add(acc, incl[lane * 8 + 7] < SAT ? incl[lane * 8 + 7] : SAT);
     }
     int ev = -1;
-    for (int k = 0; k < 512 && ev < 0; ++k) {
-      const int lane = k / 8;
-      const int live = k >= pos && k < cnt;
-      if (live && (special[k] || sat_add(excl[lane], incl[k]) >= room)) ev = k;
-    }
+    for (int k = 0; k < 512 && ev < 0; ++k)
+      if (event[k] || excl[k / 8] + (incl[k] < SAT ? incl[k] : SAT) >= room) ev = k;
     if (ev < 0) {
       s = value_of(m + acc, E);
       break;
@@ -136,9 +135,9 @@ float chain_serial(const float* x, int64_t n) {
   return s;
 }
 
-/* est[g]: estimated chain value at the start of segment g; returns the chain, *replays the count of
-   replayed segments and *rounds the wavefront rounds they took */
-float chain_replay_stats(const float* x, int64_t n, const double* est, int64_t* replays, int64_t* rounds) {
+/* est[g]: estimated chain value at the start of segment g; lanes: of a segment's records; returns the chain,
+   *replays the count of replayed segments (the first one always is) and *rounds the wavefront rounds they took */
+float chain_replay_stats(const float* x, int64_t n, const double* est, int lanes, int64_t* replays, int64_t* rounds) {
   const int L = 512;
   int64_t nseg = (n + L - 1) / L;
   int* Ea = malloc(sizeof(int) * (nseg ? nseg : 1));
@@ -149,8 +148,8 @@ float chain_replay_stats(const float* x, int64_t n, const double* est, int64_t* 
     int64_t k0 = g * L, cnt = n - k0 < L ? n - k0 : L;
     Ea[g] = est_binade(est[g] * 0.875);
     two[g] = est_binade(est[g] * 1.015625) > Ea[g];
-    wa[g] = seg_value(x, k0, cnt, Ea[g]);
-    wb[g] = two[g] ? seg_value(x, k0, cnt, Ea[g] + 1) : (1u << 24);
+    wa[g] = seg_value(x + k0, cnt, Ea[g], lanes);
+    wb[g] = two[g] ? seg_value(x + k0, cnt, Ea[g] + 1, lanes) : (1u << 24);
   }
   float s = 0.0f;
   *replays = 0;
@@ -158,7 +157,9 @@ float chain_replay_stats(const float* x, int64_t n, const double* est, int64_t* 
   for (int64_t g = 0; g < nseg && s == s; ++g) {
     int64_t k0 = g * L, cnt = n - k0 < L ? n - k0 : L;
     int ok = 0;
-    if (s <= 0x1.fffffep127f) {
+    if (g == 0) {
+      ok = 0; /* from zero, without its record */
+    } else if (s <= 0x1.fffffep127f) {
       int E = binade(s);
       uint32_t b;
       memcpy(&b, &s, 4);
@@ -184,7 +185,7 @@ float chain_replay_stats(const float* x, int64_t n, const double* est, int64_t* 
   return s;
 }
 
-float chain_replay(const float* x, int64_t n, const double* est, int64_t* replays) {
+float chain_replay(const float* x, int64_t n, const double* est, int lanes, int64_t* replays) {
   int64_t rounds = 0;
-  return chain_replay_stats(x, n, est, replays, &rounds);
+  return chain_replay_stats(x, n, est, lanes, replays, &rounds);
 }

@@ -152,6 +152,13 @@ def test_norm_one_d_tails(seed):
     _run("CAME8bit", TAILS, seed=seed)
 
 
+@pytest.mark.parametrize("seed", range(6))
+def test_norm_one_d_tails_among_larger(seed):
+    """The same lengths through the walk and its tails (k_norm_final), which a call with a larger tensor takes; by
+    themselves the one-workgroup step, with a tail rule of its own, takes them."""
+    _run("CAME8bit", TAILS + [((40001,), "normal", F32)], seed=seed)
+
+
 MATRICES = [((2048, 2048), "latin", F32), ((256, 4096), "latin", BF16), ((64, 1000), "latin", F32),
             ((2048, 2048), "normal", F32), ((64, 20000), "normal", BF16), ((1000, 3), "normal", F32),
             ((3, 50257), "heavy", F32), ((4097, 129), "normal", BF16), ((777, 1024), "sparse", BF16),

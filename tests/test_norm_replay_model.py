@@ -1,5 +1,6 @@
 """CPU check of the parallel replay of torch's fp32 norm chains (came_amd/csrc/came8_norm.h): a C model of
-its rules (tests/native/norm_replay_model.c), segment records and the wavefront replay of a segment, must
+its rules (tests/native/norm_replay_model.c), segment records from pairs of running sums and the wavefront
+replay of a segment, must
 equal the serial chain s = fma(x, x, s) bit for bit on adversarial inputs (constant values that stall the chain, values with few significant bits that make
 rounding ties, zeros, outliers, squares that are subnormal (some exact half-units of the subnormal grid)
 or overflow, NaN, rows of very different scales), whatever the binade estimates (exact, 1% off, 50% off), and replay few segments when the
@@ -28,12 +29,15 @@ def lib(tmp_path_factory):
     so.chain_serial.restype = ctypes.c_float
     so.chain_serial.argtypes = [ctypes.c_void_p, ctypes.c_int64]
     so.chain_replay.restype = ctypes.c_float
-    so.chain_replay.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)]
+    so.chain_replay.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int,
+                                ctypes.POINTER(ctypes.c_int64)]
     so.chain_replay_stats.restype = ctypes.c_float
-    so.chain_replay_stats.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+    so.chain_replay_stats.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_int,
                                       ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_int64)]
     so.chain_serial_from.restype = ctypes.c_float
     so.chain_serial_from.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_float]
+    so.seg_value.restype = ctypes.c_uint32
+    so.seg_value.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
     so.segment_replay.restype = ctypes.c_float
     so.segment_replay.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.POINTER(ctypes.c_int64)]
     return so
@@ -88,8 +92,9 @@ def test_replay_equals_serial_chain(lib, kind, noise):
         est = np.ascontiguousarray(est)
         rep = ctypes.c_int64(0)
         a = lib.chain_serial(x.ctypes.data, n)
-        b = lib.chain_replay(x.ctypes.data, n, est.ctypes.data, ctypes.byref(rep))
-        assert np.float32(a).tobytes() == np.float32(b).tobytes(), (kind, noise, n, a, b)
+        for lanes in (64, 16):
+            b = lib.chain_replay(x.ctypes.data, n, est.ctypes.data, lanes, ctypes.byref(rep))
+            assert np.float32(a).tobytes() == np.float32(b).tobytes(), (kind, noise, n, lanes, a, b)
 
 
 def test_replays_are_few_on_realistic_chains(lib):
@@ -102,7 +107,7 @@ def test_replays_are_few_on_realistic_chains(lib):
     est = np.ascontiguousarray(np.concatenate([[0.0], np.cumsum(x.astype(np.float64) ** 2)])[::512][:nseg])
     rep = ctypes.c_int64(0)
     a = lib.chain_serial(x.ctypes.data, n)
-    b = lib.chain_replay(x.ctypes.data, n, est.ctypes.data, ctypes.byref(rep))
+    b = lib.chain_replay(x.ctypes.data, n, est.ctypes.data, 16, ctypes.byref(rep))
     assert np.float32(a).tobytes() == np.float32(b).tobytes()
     assert rep.value < 60, rep.value
 
@@ -132,7 +137,7 @@ def test_replays_on_tie_dense_chains(lib):
         est = np.ascontiguousarray(np.concatenate([[0.0], np.cumsum(x.astype(np.float64) ** 2)])[::512][:nseg])
         rep, rnd = ctypes.c_int64(0), ctypes.c_int64(0)
         a = lib.chain_serial(x.ctypes.data, n)
-        b = lib.chain_replay_stats(x.ctypes.data, n, est.ctypes.data, ctypes.byref(rep), ctypes.byref(rnd))
+        b = lib.chain_replay_stats(x.ctypes.data, n, est.ctypes.data, 16, ctypes.byref(rep), ctypes.byref(rnd))
         assert np.float32(a).tobytes() == np.float32(b).tobytes()
         assert rep.value >= 0.4 * nseg, f"chain {c}: {rep.value} of {nseg} segments replayed: not tie-dense"
         reps.append(rep.value)
@@ -176,3 +181,52 @@ def test_segment_replay_from_any_start(lib, kind):
                 got = lib.segment_replay(x.ctypes.data, cnt, float(s0), ctypes.byref(rounds))
                 same = np.float32(got).tobytes() == np.float32(want).tobytes() or (np.isnan(got) and np.isnan(want))
                 assert same, (kind, float(s0), cnt, near, got, want)
+
+
+def _scaled(x, s0, rng):
+    """x with squares of 2^-k of s0 (k in [0, 24]), or None where that is not possible."""
+    top = float(np.nanmax(np.abs(x))) if np.isfinite(x).any() else 0.0
+    if not (0 < top < np.inf):
+        return None
+    return np.ascontiguousarray((x.astype(np.float64) / top * np.sqrt(float(s0)) * 2.0 ** -rng.uniform(0, 12)).astype(np.float32))
+
+
+@pytest.mark.parametrize("lanes", [64, 16])
+@pytest.mark.parametrize("kind", KINDS)
+def test_records_do_not_depend_on_the_chain(lib, kind, lanes):
+    """A record below 2^24 is the segment's increment for every chain value of its binade that it leaves inside: the serial
+    loop from the binade's first values, from even and odd ones in it and from the last one that has room ends at the
+    start plus the record's units.  A tie, a NaN or an infinity never gives such a record."""
+    rng = np.random.default_rng(zlib.crc32(f"records/{kind}/{lanes}".encode()))
+    kept = 0
+    for s0 in _starts(rng):
+        if not (np.isfinite(s0) and s0 > 0):
+            continue
+        E = max(int(np.float32(s0).view(np.uint32)) >> 23, 1) - 127
+        for cnt in (1, 9, 64, 511, 512):
+            x = _scaled(_inputs(kind, cnt, rng), s0, rng)
+            if x is None:
+                continue
+            n = lib.seg_value(x.ctypes.data, cnt, E, lanes)
+            if not np.isfinite(x).all():
+                assert n == 1 << 24
+            if n >= 1 << 24:
+                continue
+            low = 0 if E == -126 else 1 << 23
+            last = (1 << 24) - 1 - n
+            for m in {low, low + 1, (low + last) // 2, (low + last) // 2 + 1, last - 1, last}:
+                if not low <= m <= last:
+                    continue
+                start, end = (np.uint32(((E + 126) << 23) + v).view(np.float32) for v in (m, m + n))
+                got = lib.chain_serial_from(x.ctypes.data, cnt, float(start))
+                assert np.float32(got).tobytes() == end.tobytes(), (kind, float(s0), cnt, m, n)
+                kept += 1
+    assert kept > 0 or kind in ("nan", "blocks")  # a NaN in every segment; zeros only, in one so short
+
+
+def test_records_of_no_binade_are_exceptions(lib):
+    """E = 128 (the candidate above the largest binade), and sums past the largest float under E = 127."""
+    x = np.full(512, 1e18, np.float32)
+    assert lib.seg_value(x.ctypes.data, 512, 128, 64) == 1 << 24
+    x = np.full(512, 1e19, np.float32)
+    assert lib.seg_value(x.ctypes.data, 512, 127, 64) == 1 << 24
