@@ -124,6 +124,11 @@ struct Plan {
   // small tensors, a workgroup each for the whole step, by types: up to kSmallElems elements, and larger ones
   std::map<TypeKey, WorkList> smallS, smallL;
   bool small[2] = {false, false};        // [exact clip]: those lists are the step, not the passes (small_call)
+  bool can_small = false;                // every tensor is a small one
+  bool only_small = false;               // no scratch for the passes, though small_call would take them
+  size_t full_bytes = 0;                 // the workspace that small_call's choice needs
+  // whether build_plan would make this plan for a workspace of that size
+  bool fits(size_t bytes) const { return !can_small || only_small == (bytes < full_bytes); }
   std::map<TypeKey, WorkList> upd;       // P3, tile form (fast block sizes)
   std::map<TypeKey, WorkList> updb;      // P3, band form
   std::map<TypeKey, WorkList> vecB;      // 1-D pass B (fast block sizes)
@@ -461,8 +466,9 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, size
   if (n > 0 && ts == nullptr) return fail(CAME8_EINVAL, "came8: tensors is NULL");
   if (B <= 0) return fail(CAME8_EINVAL, "came8: block_size must be > 0, got " + std::to_string(B));
   plan.dev.assign(n, DevTensor{});
-  const bool can_small = all_small(ts, n);
-  for (const bool exact : {false, true}) plan.small[exact] = can_small && (only_small || small_call(ts, n, B, exact));
+  plan.can_small = all_small(ts, n);
+  plan.only_small = only_small;
+  for (const bool exact : {false, true}) plan.small[exact] = plan.can_small && (only_small || small_call(ts, n, B, exact));
   const bool small = plan.small[false] && plan.small[true];  // no passes
   // --- scratch layout (after the plan blob; offsets relative to the scratch start) ---
   std::vector<size_t> scr_off(n, 0);
@@ -843,9 +849,13 @@ int build_plan(const came8_tensor* ts, int32_t n, int32_t B, char* ws_base, size
   off = plan.zero_off + kZeroBytes;
   plan.plan_bytes = align_up(off);
   plan.total_bytes = plan.plan_bytes + scr;
-  if (can_small && !small && plan.total_bytes > limit) {
+  plan.full_bytes = plan.total_bytes;
+  if (plan.can_small && !small && plan.total_bytes > limit) {
+    const size_t full = plan.total_bytes;
     plan = Plan{};
-    return build_plan(ts, n, B, ws_base, limit, plan, true);
+    const int rc = build_plan(ts, n, B, ws_base, limit, plan, true);
+    plan.full_bytes = full;
+    return rc;
   }
 
   if (ws_base != nullptr) {
@@ -952,15 +962,14 @@ struct CacheEntry {
 };
 
 // The inputs a plan depends on, as bytes: the descriptor count, the block size, the workspace
-// address (the plan holds pointers into the workspace) and size and the descriptors themselves.
-std::vector<uint8_t> plan_inputs(const came8_tensor* ts, int32_t n, int32_t B, const void* ws, size_t ws_bytes) {
+// address (the plan holds pointers into the workspace) and the descriptors themselves.
+std::vector<uint8_t> plan_inputs(const came8_tensor* ts, int32_t n, int32_t B, const void* ws) {
   const size_t nb = size_t(std::max(n, 0)) * sizeof(came8_tensor);
-  const int64_t head[4] = {n, B, current_device(), int64_t(ws_bytes)};  // band sizes depend on the device
-  constexpr size_t H = sizeof(head);
-  std::vector<uint8_t> v(H + sizeof(void*) + nb);
-  std::memcpy(v.data(), head, H);
-  std::memcpy(v.data() + H, &ws, sizeof(void*));
-  if (nb) std::memcpy(v.data() + H + sizeof(void*), ts, nb);
+  std::vector<uint8_t> v(24 + sizeof(void*) + nb);
+  const int64_t head[3] = {n, B, current_device()};  // band sizes depend on the device
+  std::memcpy(v.data(), head, 24);
+  std::memcpy(v.data() + 24, &ws, sizeof(void*));
+  if (nb) std::memcpy(v.data() + 24 + sizeof(void*), ts, nb);
   return v;
 }
 std::mutex g_cache_mu;
@@ -1422,8 +1431,8 @@ namespace {
 // remembered (callers ask on every step)
 int plan_size(const came8_tensor* tensors, int32_t n_tensors, int32_t block_size, size_t limit, size_t* bytes) {
   static std::mutex mu;
-  static std::map<std::vector<uint8_t>, size_t> sized;
-  const std::vector<uint8_t> k = plan_inputs(tensors, n_tensors, block_size, nullptr, limit);
+  static std::map<std::pair<std::vector<uint8_t>, size_t>, size_t> sized;
+  const auto k = std::make_pair(plan_inputs(tensors, n_tensors, block_size, nullptr), limit);
   {
     std::lock_guard<std::mutex> lk(mu);
     auto it = sized.find(k);
@@ -1480,12 +1489,13 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
   int rc = CAME8_OK;
   const auto key = std::make_pair(static_cast<const void*>(workspace), workspace_tag);
   std::vector<uint8_t> inputs;
-  if (workspace_tag) inputs = plan_inputs(tensors, n_tensors, h.block_size, workspace, workspace_bytes);
+  if (workspace_tag) inputs = plan_inputs(tensors, n_tensors, h.block_size, workspace);
   std::shared_ptr<const Plan> cached;
   if (workspace_tag) {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     auto it = g_cache.find(key);
-    if (it != g_cache.end() && it->second.plan && it->second.inputs == inputs) cached = it->second.plan;
+    if (it != g_cache.end() && it->second.plan && it->second.inputs == inputs && it->second.plan->fits(workspace_bytes))
+      cached = it->second.plan;
   }
   std::shared_ptr<Plan> built;
   if (!cached) {

@@ -1,6 +1,8 @@
 """Edge shapes of the thread-per-matrix passes, of the kernels for small and narrow tensors and of the one-workgroup step,
 each step teacher-forced against the oracle under the tolerances of test_gpu_parity.py; the one-workgroup step against the
 passes, and steps over unaligned buffers against aligned ones."""
+import ctypes
+
 import pytest
 import torch
 
@@ -180,6 +182,44 @@ def test_one_launch_where_the_passes_do_not_fit():
         out.append((ps, opt, _phases(lambda: entry(opt, ps))))
     assert "small_step" not in out[0][2] and out[1][2] == {"small_step"}
     _same_steps([(ps, [opt.state[p] for p in ps]) for ps, opt, _ in out], shapes)
+
+
+def test_workspace_sizes_of_one_plan():
+    """A workspace of more bytes than a call needs has the plan that those bytes made (what a step under capture relies
+    on); one too small for the passes has a plan without them, until it is larger again."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    lib = _lib.load()
+    ps, opt = _optimizer("CAME8bit", [(20003,), (32768,)])
+    opt.step()
+    descs, _, _ = opt._descriptors([(p, opt.state[p], p.grad) for p in ps])
+    hp = opt._group_hparams(opt.param_groups[0])
+    need = ctypes.c_size_t(0)
+    _lib.check(lib.came8_workspace_size(descs, 2, 256, ctypes.byref(need)), "came8_workspace_size")
+    ws, tag = torch.empty(2 * need.value, dtype=torch.uint8, device="cuda"), _lib.new_workspace_tag()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def step(nbytes, flags=0):
+        hp.flags = flags
+        return _phases(lambda: _lib.check(lib.came8_step(descs, 2, ctypes.byref(hp), ws.data_ptr(), nbytes, tag, stream),
+                                          "came8_step"))
+
+    assert step(need.value, _lib.CAME8_FLAG_PLAN_ONLY) == set()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        stream = torch.cuda.current_stream().cuda_stream
+        hp.flags = 0
+        _lib.check(lib.came8_step(descs, 2, ctypes.byref(hp), ws.data_ptr(), 2 * need.value, tag, stream), "came8_step")
+    graph.replay()
+    torch.cuda.synchronize()
+    del graph
+    stream = torch.cuda.current_stream().cuda_stream
+    assert "small_step" not in step(need.value)
+    assert step(need.value - 1) == {"small_step"}
+    assert "small_step" not in step(need.value)
+    with pytest.raises(RuntimeError):
+        step(1024)
+    lib.came8_release_workspace(ws.data_ptr())
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
