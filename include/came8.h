@@ -229,9 +229,10 @@ int came8_step(const came8_tensor* tensors, int32_t n_tensors, const came8_hpara
  * HIP graph capture that must not call hipMalloc, tight serving loops, harnesses that forbid
  * allocation).  No counterpart in the reference.  The workspace is a static 32 MiB array in the
  * library's code object (one per GPU, held until the process ends); the call allocates nothing.
- * Tensor lists whose workspace (came8_workspace_size) exceeds 32 MiB fail with CAME8_ESPACE.  Every
- * call on one GPU shares that GPU's array and its cached launch plan: calls that overlap on one GPU
- * (other streams, other threads) race and must be serialised by the caller.  Otherwise as
+ * Tensor lists whose workspace (came8_workspace_size) exceeds 32 MiB fail with CAME8_ESPACE, but for
+ * lists of small tensors only, which are stepped another way where less is given.  Every call on one
+ * GPU shares that GPU's array and its cached launch plan: calls that overlap on one GPU (other streams,
+ * other threads) race and must be serialised by the caller.  Otherwise as
  * came8_step with a nonzero workspace tag (the plan is rebuilt when the tensor list changes).
  */
 int came8_step_static(const came8_tensor* tensors, int32_t n_tensors, const came8_hparams* hp, void* stream);
